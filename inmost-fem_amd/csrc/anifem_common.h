@@ -76,6 +76,22 @@ struct RefTensorDev {
 __host__ __device__ inline int sym_pack(int a, int b) { return a <= b ? a + b * (b + 1) / 2 : b + a * (a + 1) / 2; }
 int get_ref_tensor(int opA, int femA, int opB, int femB, int order, bool per_point, RefTensorDev* out,
                    int face = -1);
+// The per-point reference tensor in the B-operand order of the 16x16x4 matrix
+// instructions: f[(et*ks + k)*64 + l] = R[entry 16 et + l % 16][kk =
+// 4 k + l / 16], kk over q KB values, zero beyond the table; ks, the instructions
+// along kk, is a multiple of four (the kernel's unrolling).  Entry u is ib + 256 ia = ent[u] (kNoEntry
+// past n_ent): every entry, column by column, or with `packed` (a symmetric K of
+// 6 values per point: columns of K(a, b) and K(b, a) summed) those with ib >= ia.
+// Built lazily and kept like the tensors above.
+constexpr int kNoEntry = 0xFFFF;
+struct RefFragDev {
+    const double* f64 = nullptr;
+    const float* f32 = nullptr;
+    const uint16_t* ent = nullptr;
+    int ks = 0, n_ent = 0;
+};
+inline int frag_steps(int q, int kbc) { return (q * kbc + 15) / 16 * 4; }
+int get_ref_fragments(int opA, int femA, int opB, int femB, int order, int face, bool packed, RefFragDev* out);
 // Set by entry points that must not allocate device memory: get_ref_tensor
 // then only looks tables up and fails with ANIFEM_ERR_ARG where one would
 // have to be built.

@@ -74,6 +74,20 @@ int prepare_elem_args(const anifem_op& opA, const anifem_op& opB, const anifem_t
     return prepare_args(opA, opB, D, order, -1, 0, a);
 }
 
+// K symmetric: the same 3-dimensional operator of one scalar or Piola-mapped
+// space on both sides, a NULL / SCALAR / SYMMETRIC tensor, no normal
+// contraction.
+static bool symmetric_k(const anifem_op& opA, const anifem_op& opB, const ElemArgs& a) {
+    return opA.op == opB.op && opA.fem == opB.fem && opA.ncomp == 1 && opB.ncomp == 1 &&
+           ref_dim(opA.op, opA.fem) == 3 && a.mapA == a.mapB && a.mapA < 3 && !a.dot_normal &&
+           (a.ttype == ANIFEM_TENSOR_NULL || a.ttype == ANIFEM_TENSOR_SCALAR || a.ttype == ANIFEM_TENSOR_SYMMETRIC);
+}
+
+// Per-point kernel (element_point.hip); refuses nothing: returns false in
+// *taken where element_kernel has to serve the call.
+int launch_element_point(const anifem_op& opA, const anifem_op& opB, int order, bool sym, bool fp64, ElemArgs a,
+                         hipStream_t s, bool* taken);
+
 // Tets per workgroup: as many as keep the LDS geometry tensors <= 32 KiB
 // (several workgroups per CU), at most `cap`.
 static int choose_tile(int kstride, int elem_bytes, int cap) {
@@ -84,6 +98,7 @@ static int choose_tile(int kstride, int elem_bytes, int cap) {
 
 template <int DA0, int DB0, int NCA, int NCB, typename T>
 static int launch_one(ElemArgs a, int cap, hipStream_t s) {
+    const bool piola = (a.mapA | a.mapB | a.scA | a.scB) != 0;
     const int kstride = NCA * NCB * a.q * DA0 * DB0;
     a.tile = choose_tile(kstride, (int)sizeof(T), cap);
     size_t lds = (size_t)a.tile * kstride * sizeof(T);
@@ -92,7 +107,7 @@ static int launch_one(ElemArgs a, int cap, hipStream_t s) {
     if (lds > 64 * 1024) return ANIFEM_ERR_ARG;
     const int64_t blocks = (a.n + a.tile - 1) / a.tile;
     if (blocks == 0) return ANIFEM_OK;
-    if (a.mapA | a.mapB | a.scA | a.scB)
+    if (piola)
         hipLaunchKernelGGL((element_kernel<DA0, DB0, NCA, NCB, T, true>), dim3((unsigned)blocks), dim3(kBlock), lds, s,
                            a);
     else
@@ -112,7 +127,12 @@ static int launch_nc(int ncA, int ncB, const ElemArgs& a, int cap, hipStream_t s
 }
 
 template <typename T>
-int launch_element(const anifem_op& opA, const anifem_op& opB, const ElemArgs& a, int cap, hipStream_t s) {
+int launch_element(const anifem_op& opA, const anifem_op& opB, int order, const ElemArgs& a, int cap, hipStream_t s) {
+    if (a.q > 1) {
+        bool taken = false;
+        const int rc = launch_element_point(opA, opB, order, symmetric_k(opA, opB, a), sizeof(T) == 8, a, s, &taken);
+        if (rc || taken) return rc;
+    }
     const int dA = ref_dim(opA.op, opA.fem), dB = ref_dim(opB.op, opB.fem);
     if (dA == 3 && dB == 3) return launch_nc<T, 3, 3>(opA.ncomp, opB.ncomp, a, cap, s);
     if (dA == 1 && dB == 1) return launch_nc<T, 1, 1>(opA.ncomp, opB.ncomp, a, cap, s);
@@ -258,8 +278,8 @@ extern "C" int anifem_fem3dtet_batch(anifem_op opA, anifem_op opB, const anifem_
     a.xyz = xyz;
     a.out = A_out;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (precision == ANIFEM_PREC_FP64) return launch_element<double>(opA, opB, a, 256, s);
-    if (precision == ANIFEM_PREC_FP32) return launch_element<float>(opA, opB, a, 256, s);
+    if (precision == ANIFEM_PREC_FP64) return launch_element<double>(opA, opB, order, a, 256, s);
+    if (precision == ANIFEM_PREC_FP32) return launch_element<float>(opA, opB, order, a, 256, s);
     if (precision == ANIFEM_PREC_FP16X3) return launch_element_mfma(opA, opB, a, s);
     return ANIFEM_ERR_ARG;
 }
@@ -278,8 +298,8 @@ extern "C" int anifem_fem3dface_batch(anifem_op opA, anifem_op opB, const anifem
     a.xyz = xyz;
     a.out = A_out;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (precision == ANIFEM_PREC_FP64) return launch_element<double>(opA, opB, a, 256, s);
-    if (precision == ANIFEM_PREC_FP32) return launch_element<float>(opA, opB, a, 256, s);
+    if (precision == ANIFEM_PREC_FP64) return launch_element<double>(opA, opB, order, a, 256, s);
+    if (precision == ANIFEM_PREC_FP32) return launch_element<float>(opA, opB, order, a, 256, s);
     return ANIFEM_ERR_ARG;  // the MFMA mode computes volume integrals only
 }
 

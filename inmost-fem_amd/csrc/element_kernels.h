@@ -60,6 +60,10 @@ struct ElemArgs {
     float r16_scale;
     int e0pad;
     int rds_sym;       // Rds is symmetric in (ia, ib) bit for bit (RefTensorDev::rs_sym)
+    const void* frag;  // per-point K: R in operand order (RefFragDev), or null
+    const uint16_t* ent;  // its entries
+    int ks, n_ent;     // instructions along its inner dimension, number of entries
+    int ncA, ncB;      // components
 };
 
 __device__ __forceinline__ void tet_geometry(const double P[4][3], double PSI[9], double& det) {
