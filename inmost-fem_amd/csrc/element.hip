@@ -83,6 +83,9 @@ static bool symmetric_k(const anifem_op& opA, const anifem_op& opB, const ElemAr
            (a.ttype == ANIFEM_TENSOR_NULL || a.ttype == ANIFEM_TENSOR_SCALAR || a.ttype == ANIFEM_TENSOR_SYMMETRIC);
 }
 
+// Tensors constant over each tet (element_const.hip).
+int launch_element_const(const anifem_op& opA, const anifem_op& opB, bool sym, bool fp64, const ElemArgs& a,
+                         hipStream_t s);
 // Per-point kernel (element_point.hip); refuses nothing: returns false in
 // *taken where element_kernel has to serve the call.
 int launch_element_point(const anifem_op& opA, const anifem_op& opB, int order, bool sym, bool fp64, ElemArgs a,
@@ -128,11 +131,11 @@ static int launch_nc(int ncA, int ncB, const ElemArgs& a, int cap, hipStream_t s
 
 template <typename T>
 int launch_element(const anifem_op& opA, const anifem_op& opB, int order, const ElemArgs& a, int cap, hipStream_t s) {
-    if (a.q > 1) {
-        bool taken = false;
-        const int rc = launch_element_point(opA, opB, order, symmetric_k(opA, opB, a), sizeof(T) == 8, a, s, &taken);
-        if (rc || taken) return rc;
-    }
+    const bool sym = symmetric_k(opA, opB, a);
+    if (a.q == 1) return launch_element_const(opA, opB, sym, sizeof(T) == 8, a, s);
+    bool taken = false;
+    const int rc = launch_element_point(opA, opB, order, sym, sizeof(T) == 8, a, s, &taken);
+    if (rc || taken) return rc;
     const int dA = ref_dim(opA.op, opA.fem), dB = ref_dim(opB.op, opB.fem);
     if (dA == 3 && dB == 3) return launch_nc<T, 3, 3>(opA.ncomp, opB.ncomp, a, cap, s);
     if (dA == 1 && dB == 1) return launch_nc<T, 1, 1>(opA.ncomp, opB.ncomp, a, cap, s);

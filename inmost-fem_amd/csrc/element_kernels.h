@@ -8,12 +8,11 @@
 //            then the geometry tensor K = |T| T_B^T D T_A per component block
 //            (and per quadrature point when D varies inside the tet), stored
 //            to LDS.
-//   phase 2  lanes own element entries e = ib + nfB*ia; a group of G lanes
-//            covers all entries of one tet, NG = 256/G groups walk the tile's
-//            tets.  Each lane keeps its entry's reference-tensor row in
-//            registers and reads K from LDS (a broadcast within a group for
-//            scalar spaces).  Output rows of one tet are contiguous, so a
-//            group's stores (or slot-map loads) are coalesced.
+//   phase 2  the contraction of K with the reference tensor, by the kernel:
+//            element_const_kernels.h (one carried point),
+//            element_point_kernels.h (a coefficient at the points),
+//            element_kernel below (more points than that holds) and the MFMA
+//            kernels of the split-precision mode.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -308,7 +307,9 @@ __host__ __device__ inline size_t element_scale_offset(int tile, int kstride, in
 }
 
 // Element matrices of a tile of tets, stored in T precision to a.out
-// (n_tets matrices of nfB x nfA, column-major, one after the other).
+// (n_tets matrices of nfB x nfA, column-major, one after the other), for
+// coefficients at more points than the per-point kernel holds
+// (element_point.hip).
 // PIOLA (RT0, ND0 on either side): the J map of geometry_block, and a per-tet
 // factor per basis function applied to the contracted entry,
 // A(ib, ia) = sB_ib sA_ia sum_kk K R; a separate instantiation keeps the
@@ -365,19 +366,11 @@ __global__ __launch_bounds__(kBlock) void element_kernel(ElemArgs a) {
         const int ia0 = ia % a.nfA0, ca = ia / a.nfA0;
         const int rr = ib0 + a.nfB0 * ia0;
         const int koff = (cb * NCA + ca) * a.q * KB;
-        T Rreg[KB];
-        if (a.q == 1) {
-            for (int kk = 0; kk < KB; ++kk) Rreg[kk] = R[rr * KB + kk];
-        }
         for (int t = tg; t < ntile; t += NG) {
             const T* Kt = Ks + (int64_t)t * kstride + koff;
             T acc = 0;
-            if (a.q == 1) {
-                for (int kk = 0; kk < KB; ++kk) acc += Kt[kk] * Rreg[kk];
-            } else {
-                const T* Rn = R + (int64_t)rr * a.q * KB;
-                for (int j = 0; j < a.q * KB; ++j) acc += Kt[j] * Rn[j];
-            }
+            const T* Rn = R + (int64_t)rr * a.q * KB;
+            for (int j = 0; j < a.q * KB; ++j) acc += Kt[j] * Rn[j];
             if constexpr (PIOLA) {
                 if (scaled) {
                     const double* St = Ss + (int64_t)t * ns;
