@@ -16,6 +16,7 @@ from __future__ import annotations
 import ctypes
 import os
 from dataclasses import dataclass
+from functools import lru_cache
 
 import numpy as np
 
@@ -224,11 +225,19 @@ def _ptr(a):
 def _stream_handle(stream):
     if stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # no Stream object per call
+        return raw(torch.cuda.current_device()) if raw else torch.cuda.current_stream().cuda_stream
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
 # ---- operators (Operator<OP, FemFix<FEM>> / FemVec<n, FEM>) ------------------
+@lru_cache(maxsize=None)
+def _op_sizes(op, fem, ncomp):
+    """(nfa, dim) of an operator: constants of the library."""
+    c = anifem_op(op, fem, ncomp)
+    return lib().anifem_op_nfa(c), lib().anifem_op_dim(c)
+
+
 @dataclass(frozen=True)
 class Op:
     op: int
@@ -240,11 +249,11 @@ class Op:
 
     @property
     def nfa(self):
-        return lib().anifem_op_nfa(self.c())
+        return _op_sizes(self.op, self.fem, self.ncomp)[0]
 
     @property
     def dim(self):
-        return lib().anifem_op_dim(self.c())
+        return _op_sizes(self.op, self.fem, self.ncomp)[1]
 
 
 def Operator(op, fem, ncomp=1):
@@ -279,10 +288,9 @@ def fem3dtet_batch(opA: Op, opB: Op, ttype, storage, D, order, xyz, precision=PR
     """
     import torch
     n = xyz.shape[1]
-    nfa, nfb = opA.nfa, opB.nfa
-    dt = torch.float64 if precision == PREC_FP64 else torch.float32
     if out is None:
-        out = torch.empty((n, nfa, nfb), dtype=dt, device=xyz.device)
+        dt = torch.float64 if precision == PREC_FP64 else torch.float32
+        out = torch.empty((n, opA.nfa, opB.nfa), dtype=dt, device=xyz.device)
     t = anifem_tensor(ttype, storage, _ptr(D))
     rc = lib().anifem_fem3dtet_batch(opA.c(), opB.c(), ctypes.byref(t), order, n, _ptr(xyz), precision, _ptr(out),
                                      _stream_handle(stream))
@@ -322,10 +330,9 @@ def fem3dface_batch(opA: Op, opB: Op, ttype, storage, D, order, face, xyz, dot_n
     Layouts as fem3dtet_batch."""
     import torch
     n = xyz.shape[1]
-    nfa, nfb = opA.nfa, opB.nfa
-    dt = torch.float64 if precision == PREC_FP64 else torch.float32
     if out is None:
-        out = torch.empty((n, nfa, nfb), dtype=dt, device=xyz.device)
+        dt = torch.float64 if precision == PREC_FP64 else torch.float32
+        out = torch.empty((n, opA.nfa, opB.nfa), dtype=dt, device=xyz.device)
     t = anifem_tensor(ttype, storage, _ptr(D))
     rc = lib().anifem_fem3dface_batch(opA.c(), opB.c(), ctypes.byref(t), order, face, 1 if dot_normal else 0, n,
                                       _ptr(xyz), precision, _ptr(out), _stream_handle(stream))
@@ -519,11 +526,10 @@ class Assembler:
         rhs, status).  dir_values: device FP64 (ndof) Dirichlet values of the
         flagged DOFs (None: homogeneous), applied per cell as applyDir does."""
         import torch
-        dev = torch.device("cuda", torch.cuda.current_device())
         if val is None:
-            val = torch.empty(self.nnz, dtype=torch.float64, device=dev)
+            val = torch.empty(self.nnz, dtype=torch.float64, device=torch.device("cuda", torch.cuda.current_device()))
         if rhs is None and (F is not None or dir_values is not None):
-            rhs = torch.empty(self.ndof, dtype=torch.float64, device=dev)
+            rhs = torch.empty(self.ndof, dtype=torch.float64, device=torch.device("cuda", torch.cuda.current_device()))
         tD = anifem_tensor(self.tensor_type, self.tensor_storage, _ptr(D))
         tF = anifem_tensor(self.rhs_tensor_type, self.rhs_tensor_storage, _ptr(F)) if F is not None else None
         st = anifem_status()

@@ -21,9 +21,8 @@ static int prepare_args(const anifem_op& opA, const anifem_op& opB, const anifem
                         int dot_normal, ElemArgs& a) {
     if (!op_valid(opA) || !op_valid(opB) || !D) return ANIFEM_ERR_ARG;
     if (face > 3 || (face < 0 && dot_normal)) return ANIFEM_ERR_ARG;
-    std::vector<double> pts, wts;
-    int q = rule_points(order, face, pts, wts);
-    if (q < 0) return ANIFEM_ERR_ORDER;
+    const double *pts, *wts;
+    if ((face < 0 ? quadrature(order, &pts, &wts) : triangle_quadrature(order, &pts, &wts)) < 0) return ANIFEM_ERR_ORDER;
     a.face = face < 0 ? -1 : face;
     a.dot_normal = dot_normal ? 1 : 0;
     a.nfA0 = nf_scalar(opA.fem);
