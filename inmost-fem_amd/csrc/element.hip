@@ -2,12 +2,14 @@
 // helpers shared with the fused assembly.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
 #include <vector>
 
 #include "anifem_common.h"
+#include "apply_kernels.h"
 #include "element_kernels.h"
 
 namespace anifem {
@@ -309,7 +311,7 @@ namespace anifem {
 // Operator-dependent part of ApplyArgs: IDEN / GRAD of the scalar spaces,
 // IDEN / DIV / CURL of RT0 and ND0.
 static int prepare_apply(const anifem_op& op, int q, ApplyArgs& a) {
-    if (!op_valid(op) || q < 1 || q > 96) return ANIFEM_ERR_ARG;
+    if (!op_valid(op) || q < 1 || q > kMaxApplyPoints) return ANIFEM_ERR_ARG;
     if (!fem_vector(op.fem) && op.op != ANIFEM_IDEN && op.op != ANIFEM_GRAD) return ANIFEM_ERR_ARG;
     int m = 0, sc = 0;
     space_map(op.op, op.fem, m, sc);
@@ -325,34 +327,46 @@ static int prepare_apply(const anifem_op& op, int q, ApplyArgs& a) {
     return ANIFEM_OK;
 }
 
-static int run_apply(ApplyArgs a, bool mesh, hipStream_t s) {
-    const int64_t blocks = (a.n * a.q + kBlock - 1) / kBlock;
-    if (mesh) hipLaunchKernelGGL(apply_kernel<true>, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
-    else hipLaunchKernelGGL(apply_kernel<false>, dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
-    return hipGetLastError() == hipSuccess ? ANIFEM_OK : ANIFEM_ERR_HIP;
+template <int FEM, int D>
+static int launch_points(const ApplyArgs& a, const ApplyPoints& pts, bool mesh, hipStream_t s) {
+    const int dim = a.map >= 3 ? 9 : D * a.ncomp, pc = apply_chunk(a.q, dim);
+    const size_t lds = ((size_t)pc * apply_nf0(FEM) * D + (size_t)kBlock * apply_stage_row(pc, dim)) * sizeof(double);
+    const dim3 grid((unsigned)((a.n + kBlock - 1) / kBlock));
+    if (mesh) hipLaunchKernelGGL((apply_points_kernel<FEM, D, true>), grid, dim3(kBlock), lds, s, a, pts, pc);
+    else hipLaunchKernelGGL((apply_points_kernel<FEM, D, false>), grid, dim3(kBlock), lds, s, a, pts, pc);
+    ANIFEM_HIP_CHECK(hipGetLastError());
+    return ANIFEM_OK;
 }
 
-// Reference table of op at q barycentric points, on the device, and the
-// launch of apply_kernel (the table is freed after the kernel has run).
+// op at q barycentric points xyl (host) common to all cells.
 int launch_apply(const anifem_op& op, const double* xyl, int q, ApplyArgs a, bool mesh, hipStream_t s) {
     if (!xyl) return ANIFEM_ERR_ARG;
     int rc = prepare_apply(op, q, a);
     if (rc) return rc;
     if (a.n == 0) return ANIFEM_OK;
-    std::vector<double> tab;
-    reference_table(op.op, op.fem, q, xyl, tab);
-    double* dtab = nullptr;
-    ANIFEM_HIP_CHECK(hipMalloc(&dtab, tab.size() * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(dtab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) {
-        a.tab = dtab;
-        a.X = nullptr;
-        if (run_apply(a, mesh, s)) e = hipErrorLaunchFailure;
+    ApplyPoints pts;
+    std::copy(xyl, xyl + 4 * q, pts.xyl);
+    switch (op.fem) {
+        case ANIFEM_FEM_P0:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_P0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P0, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_P1:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_P1, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P1, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_P2:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_P2, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P2, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_P3:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_P3, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P3, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_CR1:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_CR1, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_CR1, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_B2:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_B2, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_B2, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_B4:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_B4, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_B4, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_RT0:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_RT0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_RT0, 1>(a, pts, mesh, s);
+        case ANIFEM_FEM_ND0:
+            return a.d == 3 ? launch_points<ANIFEM_FEM_ND0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_ND0, 1>(a, pts, mesh, s);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(dtab);
-    ANIFEM_HIP_CHECK(e);
-    return ANIFEM_OK;
+    return ANIFEM_ERR_ARG;
 }
 }  // namespace anifem
 
@@ -367,10 +381,12 @@ extern "C" int anifem_fem3dapplyx_batch(anifem_op op, int q, int64_t n_tets, con
     a.n = n_tets;
     a.xyz = xyz;
     a.X = X;
-    a.tab = nullptr;
     a.dofs = dofs;
     a.out = opU;
-    return run_apply(a, false, static_cast<hipStream_t>(stream));
+    const int64_t blocks = (a.n * a.q + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(apply_x_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
+    ANIFEM_HIP_CHECK(hipGetLastError());
+    return ANIFEM_OK;
 }
 
 extern "C" int anifem_fem3dapply_batch(anifem_op op, const double* xyl, int q, int64_t n_tets, const double* xyz,
