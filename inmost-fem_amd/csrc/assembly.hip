@@ -24,6 +24,9 @@ int prepare_elem_args(const anifem_op& opA, const anifem_op& opB, const anifem_t
 int launch_physical_points(int order, int64_t n, const double* xyz, const double* coords, const int32_t* tetnodes,
                            int64_t nodes_stride, double* X, hipStream_t s);
 int launch_apply(const anifem_op& op, const double* xyl, int q, ApplyArgs a, bool mesh, hipStream_t s);
+size_t piola_row_bytes(int nf, int d0, bool sym, int64_t n);
+int launch_piola(int d0, bool sym, bool fp64, const BlockArgs& a, double* rows, int64_t n, size_t max_lds,
+                 hipStream_t s);
 }  // namespace anifem
 
 struct anifem_assembly {
@@ -975,9 +978,90 @@ int grow(void** buf, size_t* have, size_t need) {
     return ANIFEM_OK;
 }
 
+// The row-block lists of a context.
+void set_block_lists(const anifem_assembly* ctx, anifem::BlockArgs& a) {
+    const anifem::AssemblySetup& S = ctx->S;
+    a.n_blocks = S.n_blocks;
+    a.meta = ctx->d_blk_meta;
+    a.blk_row0 = ctx->d_blk_row0;
+    a.blk_s0 = ctx->d_blk_s0;
+    a.blk_p0 = ctx->d_blk_p0;
+    a.blk_v0 = ctx->d_blk_v0;
+    a.pair_tet = ctx->d_pair_tet;
+    a.pair_ib = ctx->d_pair_ib;
+    a.pair_pos = ctx->d_pair_pos;
+    a.pair_pos8 = ctx->d_pair_pos8;
+    a.sstart = ctx->d_sstart;
+    a.pstart = ctx->d_pstart;
+    a.signmask = ctx->d_signmask;
+    a.status = ctx->d_status;
+    a.max_values = (int)S.max_block_values;
+    a.max_pairs = (int)S.max_block_pairs;
+    a.max_slots = (int)S.max_block_slots;
+}
+
+// The status of a pass whose counts are in ctx->d_status (non-finite entries;
+// the element paths count no degenerate cells).
+int read_status(const anifem_assembly* ctx, anifem_status* status, hipStream_t s) {
+    int h[4] = {0, 0, 0, 0};
+    ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
+    ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
+    status->n_nonfinite = h[0];
+    status->n_degenerate = 0;
+    status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
+    status->reserved = 0;
+    return status->code;
+}
+
+// RT0 / ND0 with one operator on both sides and tensors constant over each
+// cell: the fused pass (piola_kernels.h).  *taken stays false for the other
+// problems, which go through element matrices.
+int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor* F, int precision, double* csr_val,
+              double* rhs, anifem_status* status, hipStream_t s, bool* taken) {
+    using namespace anifem;
+    const AssemblySetup& S = ctx->S;
+    const anifem_op &tr = ctx->prob.trial, &te = ctx->prob.test;
+    if (!fem_vector(tr.fem) || tr.op != te.op || S.max_block_pairs > kBlock) return ANIFEM_OK;
+    BlockArgs a{};
+    int rc;
+    if ((rc = prepare_elem_args(tr, te, D, ctx->prob.order, a.m))) return rc;
+    a.has_rhs = F && rhs ? 1 : 0;
+    if (a.has_rhs) {
+        const anifem_op p0{ANIFEM_IDEN, ANIFEM_FEM_P0, 1}, tb{ANIFEM_IDEN, te.fem, te.ncomp};
+        if ((rc = prepare_elem_args(p0, tb, F, ctx->prob.rhs_order, a.f))) return rc;
+    }
+    const int d0 = ref_dim(tr.op, tr.fem);
+    if (a.m.q != 1 || (a.has_rhs && a.f.q != 1) || (d0 != 1 && d0 != 3)) return ANIFEM_OK;
+    const bool sym = d0 == 3 && a.m.mapA < 3 && a.m.Rds &&
+                     (D->type == ANIFEM_TENSOR_NULL || D->type == ANIFEM_TENSOR_SCALAR ||
+                      D->type == ANIFEM_TENSOR_SYMMETRIC);
+    if ((rc = grow<double>(&ctx->d_ebuf, &ctx->ebuf_bytes, piola_row_bytes(S.nf, d0, sym, S.n_tets)))) return rc;
+    *taken = true;
+    for (ElemArgs* e : {&a.m, &a.f}) {
+        e->coef_n = S.n_tets;
+        e->coords = ctx->d_coords;
+        e->tetnodes = ctx->d_tetnodes;
+        e->nodes_stride = S.n_tets;
+    }
+    a.n_kinds = 1;
+    a.kinds[0] = KindTable{sym ? a.m.Rds : a.m.Rd, sym ? a.m.Rfs : a.m.Rf, nullptr, nullptr, a.m.nfA0, a.m.nfB0, S.nf,
+                           S.nf * S.nf, 0, 0};
+    set_block_lists(ctx, a);
+    a.val = csr_val;
+    a.rhs = rhs;
+    int max_lds = 0;
+    ANIFEM_HIP_CHECK(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device));
+    // a rhs without a load vector is zero
+    if (rhs && !a.has_rhs && (rc = fill(rhs, S.ndof, s))) return rc;
+    if ((rc = launch_piola(d0, sym, precision == ANIFEM_PREC_FP64, a, static_cast<double*>(ctx->d_ebuf), S.n_tets,
+                           (size_t)max_lds, s)))
+        return rc;
+    return status ? read_status(ctx, status, s) : ANIFEM_OK;
+}
+
 // Assembly through element matrices, for the spaces whose elements the
-// fused pass does not form (RT0 / ND0: Piola map, per-DOF factors and
-// orientation signs; one-DOF spaces): the element batch (anifem_fem3dtet_batch,
+// fused passes do not form (RT0 / ND0 with two operators or a coefficient at
+// the points; one-DOF spaces): the element batch (anifem_fem3dtet_batch,
 // the reference's runtime fem3Dtet over any operator pair, int_tet.inl:2-27)
 // on the reordered cells, then the row-block scatter of element matrices
 // (anifem_assembly_run_elements, which applies the signs of oriented DOFs)
@@ -985,11 +1069,13 @@ int grow(void** buf, size_t* have, size_t need) {
 int run_via_elements(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor* F, int precision,
                      double* csr_val, double* rhs, anifem_status* status, hipStream_t s) {
     using namespace anifem;
+    bool taken = false;
+    int rc = run_piola(ctx, D, F, precision, csr_val, rhs, status, s, &taken);
+    if (rc || taken) return rc;
     const AssemblySetup& S = ctx->S;
     const int64_t n = S.n_tets;
     const int nf = S.nf;
     const size_t esz = precision == ANIFEM_PREC_FP64 ? 8 : 4;
-    int rc;
     size_t xyz_bytes = ctx->d_xyz ? (size_t)12 * n * sizeof(double) : 0;
     void* xp = ctx->d_xyz;
     if ((rc = grow<double>(&xp, &xyz_bytes, (size_t)12 * n * sizeof(double)))) return rc;
