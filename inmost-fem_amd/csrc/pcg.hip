@@ -26,6 +26,13 @@ struct PcgState {
 
 constexpr int kRedBlocks = 2048;  // partial sums per reduction
 constexpr int kThreads = 256;
+// Workgroups of the vector updates, at most, and elements per thread loaded
+// before the step's scalars are known (one while every thread has one).  Every workgroup of the next launch
+// reads every partial sum of the last one: with 2048 of them those reads were
+// most of a vector launch (P2 at 40^3, 531,441 rows: direction 10.6 and update
+// 10.6 us against 5.7 and 9.3).
+constexpr int kVecBlocks = 512;
+constexpr int vec_per_thread(int64_t n) { return n > (int64_t)kVecBlocks * kThreads ? 4 : 1; }
 
 __device__ __forceinline__ double block_sum(double v) {
     __shared__ double sh[kThreads / 64];
@@ -311,15 +318,21 @@ __global__ __launch_bounds__(kThreads) void dir_spmv_kernel(int64_t n, const int
 // p_k is the same fma of the same operands as in dir_spmv, so both forms give
 // bitwise identical iterates; the split adds one launch and 3 vectors of row
 // traffic, and halves the gathers of the SpMV.
+template <int kVec>
 __global__ __launch_bounds__(kThreads) void direction_kernel(int64_t n, const double* z, const double* p_prev,
                                                               double* p, const double* partU, int nU, int flexible,
                                                               PcgState* st, int64_t k, int check_only, int* hdone) {
     const bool first = k == 0;
-    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    double z0 = 0, p0 = 0;
-    if (i0 < n) {
-        z0 = z[i0];
-        if (!first) p0 = p_prev[i0];
+    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    double zv[kVec], pv[kVec];
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+        const int64_t i = i0 + j * step;
+        zv[j] = pv[j] = 0;
+        if (i < n) {
+            zv[j] = z[i];
+            if (!first) pv[j] = p_prev[i];
+        }
     }
     double tot[3] = {0.0, 0.0, 0.0};  // r.r, r.z, r.z_old
     if (!first) {
@@ -352,11 +365,12 @@ __global__ __launch_bounds__(kThreads) void direction_kernel(int64_t n, const do
         st->rr = rr;
         st->it = k;
     }
-    for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const bool pre = i == i0;
-        const double zi = pre ? z0 : z[i];
-        p[i] = first ? zi : fma(beta, pre ? p0 : p_prev[i], zi);
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+        const int64_t i = i0 + j * step;
+        if (i < n) p[i] = first ? zv[j] : fma(beta, pv[j], zv[j]);
     }
+    for (int64_t i = i0 + kVec * step; i < n; i += step) p[i] = first ? z[i] : fma(beta, p_prev[i], z[i]);
 }
 
 // Entries per lane of a row that the three-launch SpMV loads ahead.
@@ -434,34 +448,45 @@ __global__ __launch_bounds__(kThreads) void spmv_pdot_kernel(int64_t n, const in
 }
 
 // Jacobi update: z = Dinv r (row-local, r updated in place)
+template <int kVec>
 __global__ __launch_bounds__(kThreads) void update_jacobi_kernel(int64_t n, double* x, double* r, double* z,
                                                                   const double* p, const double* Ap,
                                                                   const double* dinv, const double* partA, int nA,
                                                                   double* partU, const PcgState* st, int64_t k) {
-    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    double x0 = 0, p0 = 0, a0 = 0, r0 = 0, d0 = 0;
-    if (i0 < n) {
-        x0 = x[i0];
-        p0 = p[i0];
-        a0 = Ap[i0];
-        r0 = r[i0];
-        d0 = dinv[i0];
+    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    double xv[kVec], pv[kVec], av[kVec], rv[kVec], dv[kVec];
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+        const int64_t i = i0 + j * step;
+        xv[j] = pv[j] = av[j] = rv[j] = dv[j] = 0;
+        if (i < n) {
+            xv[j] = x[i];
+            pv[j] = p[i];
+            av[j] = Ap[i];
+            rv[j] = r[i];
+            dv[j] = dinv[i];
+        }
     }
     double pap[1] = {thread_partial(partA, nA)};
     if (st->done) return;
     block_sums(pap);
     const double alpha = st->rzb[k & 1] / pap[0];
     double rz = 0, rr = 0;
-    for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const bool pre = i == i0;
-        x[i] = fma(alpha, pre ? p0 : p[i], pre ? x0 : x[i]);
-        const double ri = fma(-alpha, pre ? a0 : Ap[i], pre ? r0 : r[i]);
-        const double zi = (pre ? d0 : dinv[i]) * ri;
+    auto row = [&](int64_t i, double xi, double pi, double ai, double ri, double di) {
+        x[i] = fma(alpha, pi, xi);
+        ri = fma(-alpha, ai, ri);
+        const double zi = di * ri;
         r[i] = ri;
         z[i] = zi;
         rz += ri * zi;
         rr += ri * ri;
+    };
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+        const int64_t i = i0 + j * step;
+        if (i < n) row(i, xv[j], pv[j], av[j], rv[j], dv[j]);
     }
+    for (int64_t i = i0 + kVec * step; i < n; i += step) row(i, x[i], p[i], Ap[i], r[i], dinv[i]);
     double out[2] = {rz, rr};
     block_sums(out);
     if (threadIdx.x == 0) {
@@ -976,29 +1001,29 @@ extern "C" int anifem_pcg_jacobi(int64_t n, const int64_t* row_ptr, const int32_
     double *r = work, *z = r + nv, *pb[2] = {z + nv, z + 2 * nv}, *Ap = z + 3 * nv, *dinv = Ap + nv, *part = dinv + nv;
     PcgState* st = reinterpret_cast<PcgState*>(part + 3 * kRedBlocks);
     double *partA = part, *partU = part + kRedBlocks;  // p.Ap; (r.z, r.r)
-    const unsigned vb = (unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, kRedBlocks);
+    const unsigned vb = (unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, kVecBlocks);
     // r0 = b - A x0, z0 = Dinv r0
     hipLaunchKernelGGL(jacobi_inverse_kernel, dim3(vb), dim3(kThreads), 0, s, n, row_ptr, col_idx, val, dinv);
     spmv_dispatch(n, nnz, row_ptr, col_idx, val, x, Ap, nullptr, nullptr, s);
     hipLaunchKernelGGL(init_kernel, dim3(vb), dim3(kThreads), 0, s, n, b, Ap, dinv, r, z, pb[1], part);
     hipLaunchKernelGGL(reduce_kernel, dim3(1), dim3(kThreads), 0, s, part, (int)vb, 0, st, rtol);
-    const int L = lanes_per_row(n, nnz);
+    const int L = lanes_per_row(n, nnz), kv = vec_per_thread(n);
     const bool split = nnz >= kSplitNnz;
     const int nD = resident_grid(split ? spmv_pdot_kernel_of(L) : dir_kernel_of(L), red_grid(n, L));
     int rc = run_iterations(
         maxit, st,
         [&](int64_t k, int check_only, int* hdone) {
             if (split) {
-                hipLaunchKernelGGL(direction_kernel, dim3(vb), dim3(kThreads), 0, s, n, z, pb[(k + 1) & 1], pb[k & 1],
-                                   partU, (int)vb, 0, st, k, check_only, hdone);
+                hipLaunchKernelGGL(kv == 4 ? direction_kernel<4> : direction_kernel<1>, dim3(vb), dim3(kThreads), 0, s, n, z,
+                                   pb[(k + 1) & 1], pb[k & 1], partU, (int)vb, 0, st, k, check_only, hdone);
                 if (!check_only) launch_spmv_pdot(L, nD, n, row_ptr, col_idx, val, pb[k & 1], Ap, partA, st, s);
             } else {
                 launch_dir(L, nD, n, row_ptr, col_idx, val, z, pb[(k + 1) & 1], pb[k & 1], Ap, partA, partU, (int)vb,
                            0, st, k, check_only, hdone, s);
             }
             if (!check_only)
-                hipLaunchKernelGGL(update_jacobi_kernel, dim3(vb), dim3(kThreads), 0, s, n, x, r, z, pb[k & 1], Ap,
-                                   dinv, partA, nD, partU, st, k);
+                hipLaunchKernelGGL(kv == 4 ? update_jacobi_kernel<4> : update_jacobi_kernel<1>, dim3(vb), dim3(kThreads), 0, s,
+                                   n, x, r, z, pb[k & 1], Ap, dinv, partA, nD, partU, st, k);
         },
         s);
     if (rc == ANIFEM_OK) rc = finish(n, nnz, row_ptr, col_idx, val, b, x, Ap, part, st, res, s);
