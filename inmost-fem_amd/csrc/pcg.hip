@@ -705,6 +705,235 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(int64_t n, const dou
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// ---- the whole solve in one workgroup (small systems) ----------------------
+// An iteration of a small system is a chain of latencies: two launches, each
+// reading row pointers, columns, operands and partial sums that the last launch
+// left beyond this chiplet's L2 (10.8 us at 4,913 rows).  One workgroup of 16
+// waves needs no launch: p stays in LDS, x, r, 1/diag and A p in registers (lane
+// = row, R rows per lane), and the matrix is streamed from L2 in the layout its
+// first pass writes: slices of 64 rows, as wide as their longest row in groups
+// of 8 entries; a group is four 16-byte loads of values and one of 16-bit columns
+// per lane, and the next group is in flight while one is used.  The rate at which
+// one CU reads L2 then bounds it (16^3 P1, 46,941 entries: 8.7 us an iteration with the call, from 13.2).
+// Sums run in a fixed order.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallRows = 5 * kSmallThreads;
+constexpr int kSmallChunk = 8;                // entries of a row per load group
+constexpr int kSmallChunks = 192;             // load groups of 64 rows, in all
+constexpr int64_t kSmallNnz = 48 * 1024;
+constexpr int kNotTaken = 2;                   // PcgState::done: the rows do not fit the slots
+
+// One step of a wave sum: the value CTRL lanes away (data-parallel primitive),
+// zero where there is none or the row is masked out.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_from(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the wave, in lane 63: shifts by 1, 2, 4, 8 within rows of 16, then
+// row totals handed on (no LDS traffic, a quarter of a shuffle tree's latency).
+__device__ __forceinline__ double wave_sum63(double v) {
+    v += dpp_from<0x111, 0xF>(v);
+    v += dpp_from<0x112, 0xF>(v);
+    v += dpp_from<0x114, 0xF>(v);
+    v += dpp_from<0x118, 0xF>(v);
+    v += dpp_from<0x142, 0xA>(v);  // row 15 -> rows 1, 3
+    v += dpp_from<0x143, 0xC>(v);  // lane 31 -> rows 2, 3
+    return v;
+}
+
+// NV sums over the workgroup, every thread receiving them; `sh` alternates
+// between two halves, so that one barrier per call is enough.
+template <int NV>
+__device__ __forceinline__ void small_sums(double (&v)[NV], double (*sh)[kSmallWaves], int w, int l) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const double t = wave_sum63(v[i]);
+        if (l == 63) sh[i][w] = t;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        double t[kSmallWaves];
+#pragma unroll
+        for (int j = 0; j < kSmallWaves; ++j) t[j] = sh[i][j];
+#pragma unroll
+        for (int h = kSmallWaves / 2; h > 0; h /= 2)
+#pragma unroll
+            for (int j = 0; j < h; ++j) t[j] += t[j + h];
+        v[i] = t[0];
+    }
+}
+
+template <int R>
+__global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const int64_t* __restrict__ rp,
+                                                                   const int32_t* __restrict__ ci,
+                                                                   const double* __restrict__ val,
+                                                                   const double* __restrict__ b, double* x, double rtol,
+                                                                   int64_t maxit, double* __restrict__ ev,
+                                                                   uint16_t* __restrict__ ec, PcgState* st) {
+    extern __shared__ __align__(16) double p[];  // n rounded up to whole slices
+    __shared__ double sh[2][3][kSmallWaves];
+    __shared__ int off[kSmallWaves * R + 1];  // first load group of slice i of wave w: off[w R + i]
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), l = threadIdx.x % 64;
+    int64_t q0[R];
+    int len[R];
+    // groups per slice, then their places
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int row = 64 * (w + kSmallWaves * i) + l;
+        q0[i] = row < n ? rp[row] : 0;
+        len[i] = row < n ? (int)min(rp[row + 1] - q0[i], (int64_t)kSmallChunk * (kSmallChunks + 1)) : 0;
+        int m = len[i];
+        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+        if (l == 0) off[w * R + i + 1] = (m + kSmallChunk - 1) / kSmallChunk;
+    }
+    if (threadIdx.x == 0) off[0] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int s = 0; s < kSmallWaves * R; ++s) off[s + 1] += off[s];
+    __syncthreads();
+    if (off[kSmallWaves * R] > kSmallChunks) {  // uniform
+        if (threadIdx.x == 0) st->done = kNotTaken;
+        return;
+    }
+    double xr[R], rr_[R], di[R], ap[R];
+    int g1[R];
+    double s3[3] = {0.0, 0.0, 0.0};  // r.z, r.r, b.b
+    const int g0 = __builtin_amdgcn_readfirstlane(off[w * R]);
+    double2* mv = reinterpret_cast<double2*>(ev) + (size_t)g0 * (kSmallChunk / 2) * 64 + l;
+    uint4* mc = reinterpret_cast<uint4*>(ec) + (size_t)g0 * 64 + l;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int row = 64 * (w + kSmallWaves * i) + l;
+        const int ga = __builtin_amdgcn_readfirstlane(off[w * R + i]) - g0;
+        g1[i] = __builtin_amdgcn_readfirstlane(off[w * R + i + 1]) - g0;
+        xr[i] = rr_[i] = ap[i] = 0;
+        double d = 0;
+        if (64 * (w + kSmallWaves * i) < n) p[row] = row < n ? x[row] : 0.0;
+        for (int g = ga; g < g1[i]; ++g) {
+            double v[kSmallChunk];
+            uint32_t c[kSmallChunk];
+#pragma unroll
+            for (int j = 0; j < kSmallChunk; ++j) {
+                const int e = (g - ga) * kSmallChunk + j;
+                const bool has = e < len[i];
+                c[j] = has ? (uint32_t)ci[q0[i] + e] : 0u;
+                v[j] = has ? val[q0[i] + e] : 0.0;
+                if (has && (int)c[j] == row) d = v[j];
+            }
+#pragma unroll
+            for (int j = 0; j < kSmallChunk / 2; ++j)
+                mv[(size_t)(g * (kSmallChunk / 2) + j) * 64] = make_double2(v[2 * j], v[2 * j + 1]);
+            mc[(size_t)g * 64] = make_uint4(c[0] | c[1] << 16, c[2] | c[3] << 16, c[4] | c[5] << 16, c[6] | c[7] << 16);
+        }
+        di[i] = d != 0.0 ? 1.0 / d : 1.0;
+    }
+    __syncthreads();  // p (x0); a lane reads back only the entries it wrote
+    // A p of this wave's rows.  The first group is always in flight: requested
+    // before the first product, and by the last group of every product for the
+    // next one.
+    double2 nv[kSmallChunk / 2];
+    uint4 nc;
+    auto request = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < kSmallChunk / 2; ++j) nv[j] = mv[(size_t)(g * (kSmallChunk / 2) + j) * 64];
+        nc = mc[(size_t)g * 64];
+    };
+    if (g1[R - 1] > 0) request(0);
+    auto multiply = [&]() {
+        int g = 0;
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            double s = 0;
+            for (; g < g1[i]; ++g) {
+                double2 v[kSmallChunk / 2];
+#pragma unroll
+                for (int j = 0; j < kSmallChunk / 2; ++j) v[j] = nv[j];
+                const uint32_t c[4] = {nc.x, nc.y, nc.z, nc.w};
+                request(g + 1 < g1[R - 1] ? g + 1 : 0);
+                double t = 0;
+#pragma unroll
+                for (int j = 0; j < kSmallChunk / 2; ++j) {
+                    s += v[j].x * p[c[j] & 0xFFFFu];
+                    t += v[j].y * p[c[j] >> 16];
+                }
+                s += t;
+            }
+            ap[i] = s;
+        }
+    };
+    multiply();
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int row = 64 * (w + kSmallWaves * i) + l;
+        if (row < n) {
+            const double bi = b[row];
+            xr[i] = x[row];
+            rr_[i] = bi - ap[i];
+            s3[0] += rr_[i] * (di[i] * rr_[i]);
+            s3[1] += rr_[i] * rr_[i];
+            s3[2] += bi * bi;
+        }
+    }
+    small_sums(s3, sh[0], w, l);  // its barrier also ends the reads of p
+    double rz = s3[0], rr = s3[1];
+    const double bb = s3[2] > 0 ? s3[2] : 1.0, tol2 = rtol * rtol * bb;
+    // p_0 = z_0; iteration k as in dir_spmv / update_jacobi
+    double beta = 0;
+    int64_t k = 0;
+    bool done = rr <= tol2;
+    while (!done && k < maxit) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int row = 64 * (w + kSmallWaves * i) + l;
+            if (row < n) p[row] = k == 0 ? di[i] * rr_[i] : fma(beta, p[row], di[i] * rr_[i]);
+        }
+        __syncthreads();
+        multiply();
+        double pap[1] = {0.0};
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int row = 64 * (w + kSmallWaves * i) + l;
+            if (row < n) pap[0] += ap[i] * p[row];
+        }
+        small_sums(pap, sh[1], w, l);
+        const double alpha = rz / pap[0];
+        double s2[2] = {0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int row = 64 * (w + kSmallWaves * i) + l;
+            if (row < n) {
+                xr[i] = fma(alpha, p[row], xr[i]);
+                rr_[i] = fma(-alpha, ap[i], rr_[i]);
+                s2[0] += rr_[i] * (di[i] * rr_[i]);
+                s2[1] += rr_[i] * rr_[i];
+            }
+        }
+        small_sums(s2, sh[0], w, l);
+        beta = s2[0] / rz;
+        rz = s2[0];
+        rr = s2[1];
+        ++k;
+        done = rr <= tol2;
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int row = 64 * (w + kSmallWaves * i) + l;
+        if (row < n) x[row] = xr[i];
+    }
+    if (threadIdx.x == 0) {
+        st->rr = rr;
+        st->bb = bb;
+        st->tol2 = tol2;
+        st->it = k;
+        st->done = done ? 1 : 0;
+    }
+}
+
 // Returns the number of workgroups launched (= partial sums written).
 template <int L>
 static int launch_spmv(int64_t n, const int64_t* rp, const int32_t* ci, const double* v, const double* x, double* y,
@@ -959,7 +1188,29 @@ int workspace(int slot, size_t bytes, void** out) {
     return ANIFEM_OK;
 }
 
-// Final report: the true residual ||b - A x|| from x, and the state's counters.
+// Systems the one-workgroup solver takes: rows within its LDS and registers
+// and a matrix that streams faster than two launches run: 46,941 entries of 16^3
+// P1 8.7 against 13.2 us an iteration, 51,109 of P2 at 7^3 (rows of 10 to 65, wider
+// slices) 14.9 against 14.7; at 4,437 entries 3.9 against 15.7.
+bool small_system(int64_t n, int64_t nnz) { return n <= kSmallRows && nnz <= kSmallNnz; }
+
+constexpr size_t kSmallEntries = (size_t)kSmallChunks * 64 * kSmallChunk;
+size_t small_bytes() { return kSmallEntries * (sizeof(double) + sizeof(uint16_t)); }
+
+int launch_small(int64_t n, const int64_t* rp, const int32_t* ci, const double* val, const double* b, double* x,
+                 double rtol, int64_t maxit, void* work, PcgState* st, hipStream_t s) {
+    double* ev = static_cast<double*>(work);
+    uint16_t* ec = reinterpret_cast<uint16_t*>(ev + kSmallEntries);
+    const size_t lds = (size_t)((n + 63) / 64 * 64) * sizeof(double);
+    const int rows = (int)((n + kSmallThreads - 1) / kSmallThreads);
+    auto k = rows <= 1 ? pcg_small_kernel<1> : rows <= 2 ? pcg_small_kernel<2> : pcg_small_kernel<5>;
+    hipLaunchKernelGGL(k, dim3(1), dim3(kSmallThreads), lds, s, (int)n, rp, ci, val, b, x, rtol, maxit, ev, ec, st);
+    ANIFEM_HIP_CHECK(hipGetLastError());
+    return ANIFEM_OK;
+}
+
+// Final report: the true residual ||b - A x|| from x, and the state's counters
+// (kNotTaken: the one-workgroup solver left x as it was).
 int finish(int64_t n, int64_t nnz, const int64_t* rp, const int32_t* ci, const double* v, const double* b,
            const double* x, double* Ax, double* part, const PcgState* st, anifem_pcg_result* res, hipStream_t s) {
     const unsigned vb = (unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, kRedBlocks);
@@ -978,6 +1229,7 @@ int finish(int64_t n, int64_t nnz, const int64_t* rp, const int32_t* ci, const d
         res->relres = std::sqrt(hs.rr / hs.bb);
         res->true_relres = std::sqrt(tr / hs.bb);
     }
+    if (hs.done == kNotTaken) return kNotTaken;
     return hs.done ? ANIFEM_OK : ANIFEM_ERR_NOT_CONVERGED;
 }
 
@@ -997,6 +1249,16 @@ extern "C" int anifem_pcg_jacobi(int64_t n, const int64_t* row_ptr, const int32_
     {
         const int wrc = workspace(0, sizeof(double) * (6 * nv + 3 * kRedBlocks) + sizeof(PcgState), (void**)&work);
         if (wrc) return wrc;
+    }
+    if (small_system(n, nnz)) {
+        void* mat = nullptr;
+        int src = workspace(2, small_bytes(), &mat);
+        double *Ax = work, *part = work + nv;
+        PcgState* st = reinterpret_cast<PcgState*>(part + kRedBlocks);
+        if (!src) src = launch_small(n, row_ptr, col_idx, val, b, x, rtol, maxit, mat, st, s);
+        if (!src) src = finish(n, nnz, row_ptr, col_idx, val, b, x, Ax, part, st, res, s);
+        if (src != ANIFEM_OK) (void)hipStreamSynchronize(s);  // the workspace is idle on return
+        if (src != kNotTaken) return src;
     }
     double *r = work, *z = r + nv, *pb[2] = {z + nv, z + 2 * nv}, *Ap = z + 3 * nv, *dinv = Ap + nv, *part = dinv + nv;
     PcgState* st = reinterpret_cast<PcgState*>(part + 3 * kRedBlocks);
