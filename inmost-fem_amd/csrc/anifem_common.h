@@ -97,6 +97,9 @@ int get_ref_fragments(int opA, int femA, int opB, int femB, int order, int face,
 // have to be built.
 extern thread_local bool g_ref_lookup_only;
 
+// Pinned host words of the calling thread and their device address (pcg.hip).
+int* host_words(int** dev, bool may_alloc);
+
 // Symmetric-tensor packing: D(i,j), i<=j, at i + j*(j+1)/2.
 inline int sym_index(int i, int j) { return i <= j ? i + j * (j + 1) / 2 : j + i * (i + 1) / 2; }
 

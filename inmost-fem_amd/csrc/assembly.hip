@@ -125,19 +125,53 @@ __global__ void fill_int_kernel(int* p, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
 }
-// *out = the sum of the per-workgroup degenerate counts (one workgroup).
-__global__ __launch_bounds__(anifem::kBlock) void sum_counts_kernel(const int* __restrict__ c, int64_t n, int* out) {
+// The counts of a pass for the host (one workgroup): the non-finite count, and
+// the degenerate count, summed over the geometry workgroups where each stored
+// its own (deg, n of them).  `host`: pinned words, or null (status only).
+__global__ __launch_bounds__(anifem::kBlock) void publish_counts_kernel(const int* __restrict__ deg, int64_t n, int* status,
+                                                                        int* host) {
     constexpr int B = anifem::kBlock;
     __shared__ int part[B];
     int s = 0;
-    for (int64_t i = threadIdx.x; i < n; i += B) s += c[i];
+    if (deg)
+        for (int64_t i = threadIdx.x; i < n; i += B) s += deg[i];
     part[threadIdx.x] = s;
     __syncthreads();
     for (int h = B / 2; h > 0; h /= 2) {
         if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = part[0];
+    if (threadIdx.x == 0) {
+        const int d = deg ? part[0] : status[1];
+        if (deg) status[1] = d;
+        if (host) {
+            host[0] = status[0];
+            host[1] = d;
+            __threadfence_system();
+        }
+    }
+}
+
+// The status of the pass queued last on s, counts in d_status (and deg): written
+// by a launch to the thread's pinned words (a copy of 16 bytes from device
+// memory took longer than the small passes it reports on: the 16^3 P1 assembly
+// 38.5 us with it, 30.5 without), or copied where there are none.
+int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, anifem_status* status, hipStream_t s) {
+    int* dw = nullptr;
+    volatile int* hw = anifem::host_words(&dw, may_alloc);
+    int h[4] = {0, 0, 0, 0};
+    if (hw || deg) {
+        hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(anifem::kBlock), 0, s, deg, n_deg, d_status, dw);
+        ANIFEM_HIP_CHECK(hipGetLastError());
+    }
+    if (!hw) ANIFEM_HIP_CHECK(hipMemcpyAsync(h, d_status, sizeof(h), hipMemcpyDeviceToHost, s));
+    ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
+    if (hw) h[0] = hw[0], h[1] = hw[1];
+    status->n_nonfinite = h[0];
+    status->n_degenerate = h[1];
+    status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
+    status->reserved = 0;
+    return status->code;
 }
 
 int fill(double* p, int64_t n, hipStream_t s) {
@@ -1000,19 +1034,6 @@ void set_block_lists(const anifem_assembly* ctx, anifem::BlockArgs& a) {
     a.max_slots = (int)S.max_block_slots;
 }
 
-// The status of a pass whose counts are in ctx->d_status (non-finite entries;
-// the element paths count no degenerate cells).
-int read_status(const anifem_assembly* ctx, anifem_status* status, hipStream_t s) {
-    int h[4] = {0, 0, 0, 0};
-    ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-    ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-    status->n_nonfinite = h[0];
-    status->n_degenerate = 0;
-    status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-    status->reserved = 0;
-    return status->code;
-}
-
 // RT0 / ND0 with one operator on both sides and tensors constant over each
 // cell: the fused pass (piola_kernels.h).  *taken stays false for the other
 // problems, which go through element matrices.
@@ -1056,7 +1077,7 @@ int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor*
     if ((rc = launch_piola(d0, sym, precision == ANIFEM_PREC_FP64, a, static_cast<double*>(ctx->d_ebuf), S.n_tets,
                            (size_t)max_lds, s)))
         return rc;
-    return status ? read_status(ctx, status, s) : ANIFEM_OK;
+    return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
 }
 
 // Assembly through element matrices, for the spaces whose elements the
@@ -1202,21 +1223,9 @@ int assembly_run(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tens
         ctx->timers.n_launches = (per_wg ? 1 : 2) + (rhs && !do_rhs ? 1 : 0) + (S.n_blocks > 0 ? 1 : 0);
         ctx->timers.reserved = 0;
     }
-    if (status) {
-        if (per_wg) {
-            hipLaunchKernelGGL(sum_counts_kernel, dim3(1), dim3(kBlock), 0, s, ctx->d_deg,
-                               (S.n_tets + kBlock - 1) / kBlock, ctx->d_status + 1);
-            ANIFEM_HIP_CHECK(hipGetLastError());
-        }
-        int h[4] = {0, 0, 0, 0};
-        ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-        status->n_nonfinite = h[0];
-        status->n_degenerate = h[1];
-        status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-        status->reserved = 0;
-        return status->code;
-    }
+    if (status)
+        return read_status(per_wg ? ctx->d_deg : nullptr, (S.n_tets + kBlock - 1) / kBlock, ctx->d_status, !scratch, status,
+                           s);
     return ANIFEM_OK;
 }
 
@@ -1278,17 +1287,7 @@ int anifem_assembly_run_rhs(anifem_assembly* ctx, const void* F_elem, int elem_p
                                static_cast<const float*>(F_elem), accumulate ? 1 : 0);
         ANIFEM_HIP_CHECK(hipGetLastError());
     }
-    if (status) {
-        int h[4] = {0, 0, 0, 0};
-        ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-        status->n_nonfinite = h[0];
-        status->n_degenerate = 0;
-        status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-        status->reserved = 0;
-        return status->code;
-    }
-    return ANIFEM_OK;
+    return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
 }
 
 int anifem_assembly_eval(anifem_assembly* ctx, int op, const double* xyl, int q, const double* u, double* opU,
@@ -1414,17 +1413,7 @@ int anifem_assembly_run_elements(anifem_assembly* ctx, const void* A_elem, const
         else rc = launch_elements<float, false>(ctx, a, A32, F32, lds, grid, s);
         if (rc) return rc;
     }
-    if (status) {
-        int h[4] = {0, 0, 0, 0};
-        ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-        status->n_nonfinite = h[0];
-        status->n_degenerate = 0;
-        status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-        status->reserved = 0;
-        return status->code;
-    }
-    return ANIFEM_OK;
+    return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
 }
 
 int anifem_assembly_run_plain(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor* F, double* csr_val,
@@ -1519,17 +1508,7 @@ int anifem_assembly_run_plain(anifem_assembly* ctx, const anifem_tensor* D, cons
         ctx->timers.n_launches = rhs ? 4 : 3;
         ctx->timers.reserved = 0;
     }
-    if (status) {
-        int h[4] = {0, 0, 0, 0};
-        ANIFEM_HIP_CHECK(hipMemcpyAsync(h, ctx->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-        status->n_nonfinite = h[0];
-        status->n_degenerate = 0;
-        status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-        status->reserved = 0;
-        return status->code;
-    }
-    return ANIFEM_OK;
+    return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
 }
 
 }  // extern "C"

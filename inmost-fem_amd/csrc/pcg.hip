@@ -1086,13 +1086,16 @@ void launch_update_matrix(int L, int grid, int64_t n, const int64_t* mrp, const 
 #undef ANIFEM_UPD
 }
 
-// The done flag as the host sees it: one pinned, host-mapped word per host
-// thread (allocated on the thread's first solve and held until the process
-// ends).  Null if pinned memory is unavailable; the poll then copies the state.
-int* host_done_flag(int** dev) {
+// Words that kernels write and the host reads after (or, for the solvers' done
+// flag, while) they run: one pinned, host-mapped block per host thread (64
+// bytes, allocated on the thread's first use and held until the process ends).
+// Null if pinned memory is unavailable, or if there is none yet and `may_alloc`
+// is false; the caller then copies from device memory.
+int* host_words(int** dev, bool may_alloc) {
     thread_local int* h = nullptr;
     thread_local int* d = nullptr;
     if (!h) {
+        if (!may_alloc) return *dev = nullptr;
         int* p = nullptr;
         if (hipHostMalloc((void**)&p, 64, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) !=
             hipSuccess)
@@ -1115,7 +1118,7 @@ int* host_done_flag(int** dev) {
 template <class F>
 int run_iterations(int64_t maxit, const PcgState* st, F&& enqueue, hipStream_t s) {
     int* dflag = nullptr;
-    volatile int* hflag = host_done_flag(&dflag);
+    volatile int* hflag = host_words(&dflag, true);
     if (hflag) *hflag = 0;
     const int64_t chunk = 8;
     hipEvent_t ev[2] = {nullptr, nullptr};
