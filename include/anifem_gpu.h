@@ -242,7 +242,8 @@ int anifem_assembly_create(anifem_assembly** ctx, const anifem_mesh_desc* mesh, 
  * default (anifem_assembly_create) chooses them by the entries per pair:
  * 2048 / 2048 / 256 up to 10; up to 20, 4096 / 2048 / 128 for a scalar space
  * (its pass then runs two lanes per pair) and 4096 / 3072 / 256 for a vector
- * one; 4096 / 8192 / 256 above; and 8192 / 8192 (16384 above 20) / 256 when
+ * one; 2544 / 3840 / 128 for FemVec<3, P2> with a Lame tensor per tet or constant
+ * (two lanes per pair); 4096 / 8192 / 256 above; and 8192 / 8192 (16384 above 20) / 256 when
  * one row alone exceeds those.  Returns ANIFEM_ERR_DIMS when one row alone exceeds the budgets.  No
  * reference counterpart. */
 int anifem_assembly_create_budget(anifem_assembly** ctx, const anifem_mesh_desc* mesh,

@@ -337,23 +337,34 @@ int launch_persistent(anifem_assembly* ctx, const anifem::BlockArgs& a, const T*
 
 // Persistent row-block pass for vector spaces (NC components of NF0 scalar
 // DOFs on both sides): occupancy x CUs workgroups, whole XCD groups.
-template <int DA0, int DB0, int NC, int NF0, typename T, bool LC = false>
-int launch_persistent_vec(anifem_assembly* ctx, const anifem::BlockArgs& a, const T* Kg, size_t lds, hipStream_t s) {
+template <int DA0, int DB0, int NC, int NF0, typename T, bool LC, bool SPLIT>
+int launch_persistent_vec_p(anifem_assembly* ctx, const anifem::BlockArgs& a, const T* Kg, size_t lds, hipStream_t s) {
     using namespace anifem;
     int occ = 0, n_cu = 0;
     ANIFEM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &occ, reinterpret_cast<const void*>(&row_block_persistent_vec<DA0, DB0, NC, NF0, T, LC>), kBlock, lds));
+        &occ, reinterpret_cast<const void*>(&row_block_persistent_vec<DA0, DB0, NC, NF0, T, LC, SPLIT>), kBlock, lds));
     ANIFEM_HIP_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
     int64_t G = (int64_t)std::max(occ, 1) * std::max(n_cu, 1);
     G = std::min<int64_t>(G, ctx->S.n_blocks);
     G = std::max<int64_t>(8, G / 8 * 8);
-    hipLaunchKernelGGL((row_block_persistent_vec<DA0, DB0, NC, NF0, T, LC>), dim3((unsigned)G), dim3(kBlock), lds, s,
+    hipLaunchKernelGGL((row_block_persistent_vec<DA0, DB0, NC, NF0, T, LC, SPLIT>), dim3((unsigned)G), dim3(kBlock), lds, s,
                        a, Kg);
     ANIFEM_HIP_CHECK(hipGetLastError());
     return ANIFEM_OK;
 }
 
-// Compact Lame rows (lame_kblock) for GRAD x GRAD of 3-component spaces with
+// Blocks of at most kBlock/2 pairs of P2 components with compact Lame rows take
+// two lanes per pair.
+template <int DA0, int DB0, int NC, int NF0, typename T, bool LC = false>
+int launch_persistent_vec(anifem_assembly* ctx, const anifem::BlockArgs& a, const T* Kg, size_t lds, hipStream_t s) {
+    if constexpr (NF0 == 10 && LC) {
+        if (ctx->S.max_block_pairs <= anifem::kBlock / 2)
+            return launch_persistent_vec_p<DA0, DB0, NC, NF0, T, LC, true>(ctx, a, Kg, lds, s);
+    }
+    return launch_persistent_vec_p<DA0, DB0, NC, NF0, T, LC, false>(ctx, a, Kg, lds, s);
+}
+
+// Compact Lame rows (lame_row) for GRAD x GRAD of 3-component spaces with
 // the Lame tensor constant over each tet, volume integrals.
 template <int NCA, int NCB, int KDA, int KDB>
 bool lame_compact(const anifem::BlockArgs& a) {
@@ -637,13 +648,16 @@ int build_host(anifem_assembly* ctx, const anifem_mesh_desc* mesh, const anifem_
     ctx->prob = *prob;
     ctx->prob.dirichlet_dof_mask = nullptr;
     const int nf = nf_scalar(prob->test.fem) * prob->test.ncomp;
-    const BlockCaps c = caps ? *caps : default_caps(nf, prob->test.ncomp == 1);
-    const int rc =
-        on_device ? build_setup_device(*mesh, *prob, ctx->S, c, stream) : build_setup(*mesh, *prob, ctx->S, c);
-    if (rc != ANIFEM_ERR_DIMS || caps) return rc;
-    ctx->S = AssemblySetup();  // the default budgets, then wider ones when one row exceeds them
-    const BlockCaps w = wide_caps(nf);
-    return on_device ? build_setup_device(*mesh, *prob, ctx->S, w, stream) : build_setup(*mesh, *prob, ctx->S, w);
+    auto build = [&](const BlockCaps& c) {
+        return on_device ? build_setup_device(*mesh, *prob, ctx->S, c, stream) : build_setup(*mesh, *prob, ctx->S, c);
+    };
+    if (caps) return build(*caps);
+    int rc = ANIFEM_ERR_DIMS;
+    for (const BlockCaps& c : caps_ladder(nf, *prob, false)) {
+        ctx->S = AssemblySetup();
+        if ((rc = build(c)) != ANIFEM_ERR_DIMS) break;
+    }
+    return rc;
 }
 
 }  // namespace
@@ -658,10 +672,11 @@ namespace {
 int create_default(anifem_assembly** out, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob, int nf,
                    void* stream, const anifem_vars_desc* vars) {
     using namespace anifem;
-    const bool scalar_space = !vars && prob->test.ncomp == 1;
-    const int rc = assembly_create_caps(out, mesh, prob, default_caps(nf, scalar_space), stream, vars);
-    if (rc != ANIFEM_ERR_DIMS) return rc;
-    return assembly_create_caps(out, mesh, prob, wide_caps(nf), stream, vars);
+    if (!prob) return ANIFEM_ERR_ARG;
+    int rc = ANIFEM_ERR_DIMS;
+    for (const BlockCaps& c : caps_ladder(nf, *prob, vars != nullptr))
+        if ((rc = assembly_create_caps(out, mesh, prob, c, stream, vars)) != ANIFEM_ERR_DIMS) break;
+    return rc;
 }
 }  // namespace
 

@@ -64,7 +64,7 @@ struct BlockArgs {
     const uint16_t* sstart;     // per slot: first value, relative to its block
     const uint16_t* pstart;     // per row: first pair, relative to its block
     const uint64_t* signmask;   // element-matrix passes: per tet, bit j = local DOF j has orientation sign -1, or null
-    int lamec;                  // geometry rows hold the compact Lame form (lame_kblock), not the K blocks
+    int lamec;                  // geometry rows hold the compact Lame form (lame_row), not the K blocks
     double* val;
     double* rhs;
     int* status;
@@ -146,35 +146,74 @@ __device__ __forceinline__ void tri_copy(V* __restrict__ dst, const V* __restric
 // entries of T^T C T collapses to
 //   K_(cb,ca)(b, a) = lam T(cb,b) T(ca,a) + mu (d_{cb,ca} (T^T T)(b,a) + T(ca,b) T(cb,a)),
 // lam and mu scaled by the cell measure.  A compact row holds Tm, lam, mu
-// (kLameCompact values) instead of the 81 values of the nine blocks; every
-// pass expands the blocks it needs with this function, with its roundings
-// fixed (no contraction left to the compiler), so all passes agree bitwise.
+// (kLameCompact values) instead of the 81 values of the nine blocks.
+// The entry of component ca against a reference row r(b, a) needs no block:
+//   sum_{b,a} K(b, a) r(b, a) = T(ca, .) . z + d_{cb,ca} g,
+//   z_k = lam sum_b T(cb,b) r(b,k) + mu sum_a T(cb,a) r(k,a),  g = mu sum (T^T T) r,
+// z and g shared by the three components: 36 products per reference row in
+// place of 27 and the expansion of the 27 block values, and 21 values held per
+// pair in place of 41.  Every pass forms its entries with these functions,
+// with the roundings fixed (no contraction left to the compiler), so all passes
+// agree bitwise.
 constexpr int kLameCompact = 11;
 
-// u = row cb of T, v = row ca, same = (cb == ca); callers read u and v from
-// the row (or from c with fixed indices): a runtime index into a register
-// array would move the array to scratch memory.
 template <typename T>
-__device__ __forceinline__ void lame_kblock(const T* c, const T* u, const T* v, bool same, T* Kb) {
+struct LameRow {
+    T ul[3], um[3];  // lam and mu times row cb of T
+    T g[6];          // mu T^T T, packed (sym_pack)
+};
+
+// c: the compact row; u: row cb of its T (callers read it by address: a runtime
+// index into a register array would move the array to scratch memory).
+template <typename T>
+__device__ __forceinline__ LameRow<T> lame_row(const T* c, const T* u) {
 #pragma clang fp contract(off)
-    const T lam = c[9], mu = c[10];
+    LameRow<T> L;
 #pragma unroll
-    for (int b = 0; b < 3; ++b)
+    for (int k = 0; k < 3; ++k) {
+        L.ul[k] = c[9] * u[k];
+        L.um[k] = c[10] * u[k];
+    }
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            T e = lam * (u[b] * v[a]);
-            e = fma(mu, v[b] * u[a], e);
-            const T g = fma(c[b + 6], c[a + 6], fma(c[b + 3], c[a + 3], c[b] * c[a]));
-            const T eg = fma(mu, g, e);
-            Kb[b * 3 + a] = same ? eg : e;
-        }
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b <= a; ++b) L.g[sym_pack(b, a)] = c[10] * fma(c[b + 6], c[a + 6], fma(c[b + 3], c[a + 3], c[b] * c[a]));
+    return L;
 }
 
-// The (cb, ca) block of a compact row in global memory, contracted with one
-// reference row r of 9 values (the contraction order of the row-block passes).
+// z and g of one reference row of 9 values.
+template <typename T>
+__device__ __forceinline__ void lame_contract(const LameRow<T>& L, const T* r, T* z, T& g) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        T t = L.ul[0] * r[k];
+        t = fma(L.ul[1], r[3 + k], t);
+        t = fma(L.ul[2], r[6 + k], t);
+        t = fma(L.um[0], r[3 * k], t);
+        t = fma(L.um[1], r[3 * k + 1], t);
+        z[k] = fma(L.um[2], r[3 * k + 2], t);
+    }
+    T t = L.g[0] * r[0];
+    t = fma(L.g[2], r[4], t);
+    t = fma(L.g[5], r[8], t);
+    t = fma(L.g[1], r[1] + r[3], t);
+    t = fma(L.g[3], r[2] + r[6], t);
+    g = fma(L.g[4], r[5] + r[7], t);
+}
+
+// The entry of the component whose row of T is v; same: it is the pair's own.
+template <typename T>
+__device__ __forceinline__ T lame_value(const T* v, const T* z, T g, bool same) {
+#pragma clang fp contract(off)
+    const T e = fma(v[2], z[2], fma(v[1], z[1], v[0] * z[0]));
+    return same ? e + g : e;
+}
+
+// The (cb, ca) entry of a compact row in global memory against one reference row.
 template <typename T>
 __device__ __forceinline__ T lame_entry(const T* Kt, int cb, int ca, const T* r) {
-    T c[kLameCompact], u[3], v[3], kb[9];
+    T c[kLameCompact], u[3], v[3], z[3], g;
 #pragma unroll
     for (int j = 0; j < kLameCompact; ++j) c[j] = Kt[j];
 #pragma unroll
@@ -182,11 +221,8 @@ __device__ __forceinline__ T lame_entry(const T* Kt, int cb, int ca, const T* r)
         u[k] = Kt[3 * cb + k];
         v[k] = Kt[3 * ca + k];
     }
-    lame_kblock(c, u, v, cb == ca, kb);
-    T acc = 0;
-#pragma unroll
-    for (int j = 0; j < 9; ++j) acc += kb[j] * r[j];
-    return acc;
+    lame_contract(lame_row(c, u), r, z, g);
+    return lame_value(v, z, g, cb == ca);
 }
 
 // Geometry pass over all tets (one lane per tet): FP64 Jacobian, inverse and
@@ -204,7 +240,7 @@ __host__ __device__ inline size_t geometry_stage_bytes(int rowlen) {
     return ((NCA * NCB == 1 || LC) && rowlen <= 16) ? (size_t)kBlock * rowlen * sizeof(T) : 0;
 }
 
-// LC: compact Lame rows (lame_kblock; a tensor constant over each tet).
+// LC: compact Lame rows (lame_row; a tensor constant over each tet).
 template <int DA0, int DB0, int NCA, int NCB, typename T, bool SYM = false, bool LC = false>
 __global__ __launch_bounds__(kBlock) void geometry_kernel(BlockArgs a, T* __restrict__ Kg, int64_t n_tets) {
     static_assert(!SYM || (DA0 == 3 && DB0 == 3 && NCA == 1 && NCB == 1), "packed K: 3 x 3 scalar blocks");
@@ -376,15 +412,17 @@ __global__ __launch_bounds__(kBlock) void row_block_kernel(BlockArgs a, const T*
     const T* Kt = Kg + (int64_t)tet * a.rowlen;
     const bool qc = len == KB;  // one carried point: K blocks held in registers
     T kreg[NCA][KB];
-    if constexpr (NCA == 3 && NCB == 3 && KB == 9) {
-        if (a.lamec) {  // compact Lame row: the pair's three blocks in closed form
-            T c[kLameCompact], u[3];
+    constexpr bool kLame = NCA == 3 && NCB == 3 && KB == 9;
+    T lc[kLame ? kLameCompact : 1];  // compact Lame row of the pair's cell
+    LameRow<T> lr;
+    if constexpr (kLame) {
+        if (a.lamec) {
+            T u[3];
 #pragma unroll
-            for (int j = 0; j < kLameCompact; ++j) c[j] = has_pair ? Kt[j] : T(0);
+            for (int j = 0; j < kLameCompact; ++j) lc[j] = has_pair ? Kt[j] : T(0);
 #pragma unroll
             for (int k = 0; k < 3; ++k) u[k] = has_pair ? Kt[3 * cb + k] : T(0);
-#pragma unroll
-            for (int ca = 0; ca < NCA; ++ca) lame_kblock(c, u, c + 3 * ca, cb == ca, kreg[ca]);
+            lr = lame_row(lc, u);
         }
     }
     if (qc && !a.lamec) {
@@ -440,10 +478,16 @@ __global__ __launch_bounds__(kBlock) void row_block_kernel(BlockArgs a, const T*
         const bool dir = (ibf & kPairDirichlet) != 0;
         const int ib0 = ib % nfB0;
         const uint16_t* pos = a.pair_pos + qp;
-        auto entry = [&](int ps, const T* Kb, const T* kr, int ia0) {
+        auto entry = [&](int ps, const T* Kb, const T* kr, int ca, int ia0) {
             const T* Rr = R + (ib0 + nfB0 * ia0) * rstride;
             T acc = 0;
-            if (qc) {
+            if (kLame && a.lamec) {
+                if constexpr (kLame) {
+                    T z[3], g;
+                    lame_contract(lr, Rr, z, g);
+                    acc = lame_value(lc + 3 * ca, z, g, ca == cb);
+                }
+            } else if (qc) {
 #pragma unroll
                 for (int j = 0; j < KB; ++j) acc += kr[j] * Rr[j];
             } else {
@@ -460,14 +504,14 @@ __global__ __launch_bounds__(kBlock) void row_block_kernel(BlockArgs a, const T*
             for (int ia0 = 0; ia0 < 2 * PW; ++ia0) {
                 const uint32_t w = posw[ia0 >> 1];
                 const int ps = (int)((ia0 & 1) ? (w >> 16) : (w & 0xFFFFu));
-                if (ia0 < nfA0 && ps != kPosDropped) entry(ps, Kt + cb * len, kreg[0], ia0);
+                if (ia0 < nfA0 && ps != kPosDropped) entry(ps, Kt + cb * len, kreg[0], 0, ia0);
             }
         } else {
 #pragma unroll
             for (int ca = 0; ca < NCA; ++ca) {
                 for (int ia0 = 0; ia0 < nfA0; ++ia0) {
                     const int ps = pos[ca * nfA0 + ia0];
-                    if (ps != kPosDropped) entry(ps, Kt + (cb * NCA + ca) * len, kreg[ca], ia0);
+                    if (ps != kPosDropped) entry(ps, Kt + (cb * NCA + ca) * len, kreg[ca], ca, ia0);
                 }
             }
         }
@@ -1059,16 +1103,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
 // registers (no occupancy cap on the register count), which is what hides
 // the gather latency.  Same arithmetic and summation order as
 // row_block_kernel: the results are bitwise identical.
-// LC: compact Lame rows; a pair carries 11 values and expands its three
-// blocks in phase A (lame_kblock).
-template <int DA0, int DB0, int NC, int NF0, typename T, bool LC = false>
-__global__ __launch_bounds__(kBlock) void row_block_persistent_vec(BlockArgs a, const T* __restrict__ Kg) {
+// LC: compact Lame rows; a pair carries 11 values and its own row of T
+// (lame_row).
+// SPLIT (blocks of at most kBlock/2 pairs): two lanes per pair, lane t and lane
+// t + kBlock/2 forming the columns ia0 < NF0/2 and >= NF0/2 of every component:
+// every lane works in phase A on a block half as large, and the shorter position
+// lists and slot starts let three waves per SIMD (three workgroups per CU) hide
+// the gathers instead of two.  Same values and sums.  Elasticity on the 48^3
+// cube: pass in FP64 1.69 -> 1.60 ms, in FP32 1.57 -> 1.25; blocks of 102 and 111
+// pairs at four waves 1.64 and 1.61, of 256 pairs and one lane 1.77.
+template <int DA0, int DB0, int NC, int NF0, typename T, bool LC = false, bool SPLIT = false>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 1))) void row_block_persistent_vec(BlockArgs a, const T* __restrict__ Kg) {
     static_assert(!LC || (NC == 3 && DA0 == 3 && DB0 == 3), "compact Lame rows: FemVec<3> gradients");
     constexpr int KB = DA0 * DB0;
     constexpr int NF = NC * NF0;       // entries per pair
-    constexpr int PW = NF / 2;         // position words per pair
+    static_assert(!SPLIT || (NF0 == 10 && LC), "split pairs: halves of five columns, compact Lame rows");
+    constexpr int HC = SPLIT ? NF0 / 2 : NF0;  // columns per lane and component
+    constexpr int CW = SPLIT ? 3 : NF0 / 2;    // position words per lane and component
+    constexpr int PW = SPLIT ? NC * CW : NF / 2;  // position words per lane
+    constexpr int kHalf = kBlock / 2;
+    const int pl = SPLIT ? ((int)threadIdx.x & (kHalf - 1)) : (int)threadIdx.x;  // the lane's pair
+    const int half = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kHalf) : 0;
     static_assert(NF % 2 == 0, "positions are read as 32-bit words");
-    constexpr int SW = 9;              // slot-start words per lane: blocks of at most 4606 slots
+    constexpr int SW = SPLIT ? 5 : 9;  // slot-start words per lane: blocks of at most 2558 or 4606 slots
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lenp = pad16<T>(KB);
     const int lenFp = a.has_rhs ? pad16<T>(1) : 0;
@@ -1111,18 +1168,18 @@ __global__ __launch_bounds__(kBlock) void row_block_persistent_vec(BlockArgs a, 
         int pst;
     };
     auto load_records = [&](const BlockMeta& Mx, Regs& P) {
-        const bool hp = (int)threadIdx.x < Mx.np;
-        const int64_t gp = Mx.p0 + (hp ? threadIdx.x : 0);
+        const bool hp = pl < Mx.np;
+        const int64_t gp = Mx.p0 + (hp ? pl : 0);
         P.tet = hp ? a.pair_tet[gp] : 0;
         P.ibf = hp ? a.pair_ib[gp] : 0;
         // NF even: a pair's positions start at an even entry (q0 = p0 * NF)
         const uint32_t* pw =
-            reinterpret_cast<const uint32_t*>(a.pair_pos + Mx.q0 + (int64_t)(hp ? threadIdx.x : 0) * NF);
+            reinterpret_cast<const uint32_t*>(a.pair_pos + Mx.q0 + (int64_t)(hp ? pl : 0) * NF) + 2 * half;
 #pragma unroll
-        for (int w = 0; w < PW; ++w) P.posw[w] = hp ? pw[w] : 0u;
+        for (int w = 0; w < PW; ++w) P.posw[w] = hp ? pw[SPLIT ? w / CW * (NF0 / 2) + w % CW : w] : 0u;
     };
     auto load_k = [&](const BlockMeta& Mx, Regs& P) {
-        const bool hp = (int)threadIdx.x < Mx.np;
+        const bool hp = pl < Mx.np;
         const int cb = (P.ibf & 63) / NF0;
         const T* Kt = Kg + (int64_t)P.tet * a.rowlen;
         if constexpr (LC) {
@@ -1182,42 +1239,55 @@ __global__ __launch_bounds__(kBlock) void row_block_persistent_vec(BlockArgs a, 
         if (bnn >= 0) Mnn = a.meta[bnn];
 
         // phase A of b: entries (ib, ca*NF0 + ia0) of the pair's row
-        if ((int)threadIdx.x < M.np) {
+        if (pl < M.np) {
             const int ib = cur.ibf & 63;
             const int ib0 = ib % NF0;
             const bool dir = (cur.ibf & kPairDirichlet) != 0;
             const T* Rb = R + ib0 * lenp;
-            T kx[LC ? NC : 1][LC ? KB : 1];  // the expanded blocks of a compact row
-            if constexpr (LC) {
+            const int cb = ib / NF0;
+            LameRow<T> lr;
+            if constexpr (LC) lr = lame_row(cur.c, cur.u);
+            // one reference row per ia0, shared by the NC component entries;
+            // columns IA .. IA + HC - 1 (IA = 0, or HC on the second lane of a
+            // split pair, whose words start one position early)
+            auto columns = [&](auto ia_c) {
+                constexpr int IA = decltype(ia_c)::value;
 #pragma unroll
-                for (int ca = 0; ca < NC; ++ca) lame_kblock(cur.c, cur.u, cur.c + 3 * ca, ib / NF0 == ca, kx[ca]);
-            }
-            // one reference row per ia0, shared by the NC component entries
+                for (int i = 0; i < HC; ++i) {
+                    T r[KB];
 #pragma unroll
-            for (int ia0 = 0; ia0 < NF0; ++ia0) {
-                T r[KB];
+                    for (int j = 0; j < KB; ++j) r[j] = Rb[NF0 * (IA + i) * lenp + j];
+                    T z[3], g = 0;
+                    if constexpr (LC) lame_contract(lr, r, z, g);
 #pragma unroll
-                for (int j = 0; j < KB; ++j) r[j] = Rb[NF0 * ia0 * lenp + j];
+                    for (int ca = 0; ca < NC; ++ca) {
+                        const int e = SPLIT ? i + (IA & 1) : i;  // position within the component's words
+                        const uint32_t w = cur.posw[ca * CW + (e >> 1)];
+                        const int ps = (int)((e & 1) ? (w >> 16) : (w & 0xFFFFu));
+                        if (ps != kPosDropped) {
+                            T acc = 0;
+                            if constexpr (LC) {
+                                acc = lame_value(cur.c + 3 * ca, z, g, ca == cb);
+                            } else {
 #pragma unroll
-                for (int ca = 0; ca < NC; ++ca) {
-                    const int e = ca * NF0 + ia0;
-                    const uint32_t w = cur.posw[e >> 1];
-                    const int ps = (int)((e & 1) ? (w >> 16) : (w & 0xFFFFu));
-                    if (ps != kPosDropped) {
-                        T acc = 0;
-#pragma unroll
-                        for (int j = 0; j < KB; ++j) acc += (LC ? kx[LC ? ca : 0][LC ? j : 0] : cur.k[LC ? 0 : ca][LC ? 0 : j]) * r[j];
-                        const double v = dir ? 1.0 : (double)acc;
-                        nonfinite += isfinite(v) ? 0 : 1;
-                        vals[ps] = v;
+                                for (int j = 0; j < KB; ++j) acc += cur.k[ca][j] * r[j];
+                            }
+                            const double v = dir ? 1.0 : (double)acc;
+                            nonfinite += isfinite(v) ? 0 : 1;
+                            vals[ps] = v;
+                        }
                     }
                 }
-            }
-            if (a.has_rhs) {
+            };
+            if (SPLIT && half)  // uniform over each wave
+                columns(std::integral_constant<int, SPLIT ? HC : 0>{});
+            else
+                columns(std::integral_constant<int, 0>{});
+            if (a.has_rhs && half == 0) {
                 const T acc = cur.kf * RF[ib0 * lenFp];
                 const double fv = dir ? 0.0 : (double)acc;
                 nonfinite += isfinite(fv) ? 0 : 1;
-                fvals[threadIdx.x] = fv;
+                fvals[pl] = fv;
             }
         }
         // geometry rows, slot and row starts of the next block

@@ -39,12 +39,39 @@ inline BlockCaps default_caps(int nf, bool scalar_space) {
     }
     return c;
 }
+// Elasticity on three components of P2 (30 entries per pair, the compact Lame
+// rows) takes blocks of 128 pairs as well: two lanes per pair in the fused pass and
+// three workgroups per CU instead of two (48^3 cube: FP64 1.69 -> 1.60 ms, FP32
+// 1.57 -> 1.25).  The scatter of element matrices on these blocks went from 3.37 to
+// 2.59 ms (FP64 symmetric), 2.94 to 1.89 (FP32 symmetric), 4.41 to 4.08 (FP32
+// general) and 5.51 to 5.67 (FP64 general: whole-row gathers); other tensors, whose
+// pass holds the blocks of K in registers and stays at two workgroups, keep the
+// budgets of default_caps.  The slots stay within what the pass carries in
+// registers.
+inline BlockCaps p2vec_caps() {
+    BlockCaps c;
+    c.max_slots = 2544;
+    c.max_values = 3840;
+    c.max_pairs = 128;
+    return c;
+}
 // Budgets for a mesh one of whose rows exceeds default_caps (a node with
 // more incident cells than the default blocks hold: with P3, more than 102).
 inline BlockCaps wide_caps(int nf) {
     BlockCaps c;
     c.max_slots = 8192;
     c.max_values = nf > 20 ? 16384 : 8192;
+    return c;
+}
+// The budgets to try in turn, each where a single row exceeds the one before.
+inline std::vector<BlockCaps> caps_ladder(int nf, const anifem_problem_desc& prob, bool vars) {
+    const int ncomp = vars ? 0 : prob.test.ncomp;  // several variables: the budgets of a vector space
+    std::vector<BlockCaps> c;
+    if (nf == 30 && ncomp == 3 && prob.tensor_type == ANIFEM_TENSOR_LAME &&
+        prob.tensor_storage != ANIFEM_COEF_PER_POINT)
+        c.push_back(p2vec_caps());
+    c.push_back(default_caps(nf, ncomp == 1));
+    c.push_back(wide_caps(nf));
     return c;
 }
 constexpr uint16_t kPosDropped = 0xFFFF;  // pair_pos of an entry the pattern drops
