@@ -11,6 +11,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
+#include <new>
+#include <utility>
 #include <vector>
 
 #include "anifem_common.h"
@@ -1087,27 +1090,64 @@ void launch_update_matrix(int L, int grid, int64_t n, const int64_t* mrp, const 
 }
 
 // Words that kernels write and the host reads after (or, for the solvers' done
-// flag, while) they run: one pinned, host-mapped block per host thread (64
-// bytes, allocated on the thread's first use and held until the process ends).
-// Null if pinned memory is unavailable, or if there is none yet and `may_alloc`
-// is false; the caller then copies from device memory.
-int* host_words(int** dev, bool may_alloc) {
-    thread_local int* h = nullptr;
-    thread_local int* d = nullptr;
-    if (!h) {
-        if (!may_alloc) return *dev = nullptr;
-        int* p = nullptr;
-        if (hipHostMalloc((void**)&p, 64, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) !=
-            hipSuccess)
-            return *dev = nullptr;
-        if (hipHostGetDevicePointer((void**)&d, p, 0) != hipSuccess) {
-            (void)hipHostFree(p);
-            return *dev = nullptr;
-        }
-        h = p;
+// flag, while) they run: one pinned, host-mapped block of 64 bytes per host
+// thread, taken on the thread's first use and handed to a later thread when it
+// ends, so there are never more than threads alive at once.  Every user waits
+// for its stream before it returns.  Null if pinned memory is unavailable, or
+// if the thread has none yet and `may_alloc` is false; the caller then copies
+// from device memory.
+struct HostWords {
+    int* h = nullptr;
+    int* d = nullptr;
+    ~HostWords();
+};
+struct HostWordsPool {
+    std::mutex m;
+    std::vector<std::pair<int*, int*>> idle;
+};
+HostWordsPool& host_words_pool() {
+    static HostWordsPool* p = new HostWordsPool;  // outlives every thread's words
+    return *p;
+}
+HostWords::~HostWords() {
+    if (!h) return;
+    HostWordsPool& p = host_words_pool();
+    std::lock_guard<std::mutex> lock(p.m);
+    try {
+        p.idle.emplace_back(h, d);
+    } catch (const std::bad_alloc&) {  // not handed on
     }
-    *dev = d;
-    return h;
+}
+
+int* host_words(int** dev, bool may_alloc) {
+    thread_local HostWords w;
+    if (!w.h) {
+        *dev = nullptr;
+        if (!may_alloc) return nullptr;
+        {
+            HostWordsPool& pool = host_words_pool();
+            std::lock_guard<std::mutex> lock(pool.m);
+            if (!pool.idle.empty()) {
+                w.h = pool.idle.back().first;
+                w.d = pool.idle.back().second;
+                pool.idle.pop_back();
+            }
+        }
+        if (!w.h) {
+            int *p = nullptr, *d = nullptr;
+            if (hipHostMalloc((void**)&p, 64, hipHostMallocMapped | hipHostMallocCoherent | hipHostMallocPortable) !=
+                hipSuccess)
+                return nullptr;
+            if (hipHostGetDevicePointer((void**)&d, p, 0) != hipSuccess) {
+                (void)hipHostFree(p);
+                return nullptr;
+            }
+            w.h = p;
+            w.d = d;
+        }
+    }
+    *dev = w.d;
+    return w.h;
 }
 
 // Queue the iterations in chunks; after queueing chunk c, wait for chunk c-1
@@ -1165,7 +1205,7 @@ struct WorkEntry {
     void* p;
     size_t bytes;
 };
-constexpr int kWorkEntries = 16;
+constexpr int kWorkEntries = 24;  // three slots on each of eight devices
 thread_local WorkEntry tl_work[kWorkEntries];
 thread_local int tl_work_used = 0;
 
@@ -1255,7 +1295,11 @@ extern "C" int anifem_pcg_jacobi(int64_t n, const int64_t* row_ptr, const int32_
     }
     if (small_system(n, nnz)) {
         void* mat = nullptr;
-        int src = workspace(2, small_bytes(), &mat);
+        int src = ANIFEM_OK;
+        if (workspace(2, small_bytes(), &mat)) {  // no room for the padded matrix: the launches below need none
+            (void)hipGetLastError();
+            src = kNotTaken;
+        }
         double *Ax = work, *part = work + nv;
         PcgState* st = reinterpret_cast<PcgState*>(part + kRedBlocks);
         if (!src) src = launch_small(n, row_ptr, col_idx, val, b, x, rtol, maxit, mat, st, s);
