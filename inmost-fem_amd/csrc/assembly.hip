@@ -1068,11 +1068,12 @@ int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor*
     }
     const int d0 = ref_dim(tr.op, tr.fem);
     if (a.m.q != 1 || (a.has_rhs && a.f.q != 1) || (d0 != 1 && d0 != 3)) return ANIFEM_OK;
-    const bool sym = d0 == 3 && a.m.mapA < 3 && a.m.Rds &&
+    // packed in FP64 only: the column sums of R would round FP32 entries another
+    // way than the element matrices of that mode
+    const bool sym = precision == ANIFEM_PREC_FP64 && d0 == 3 && a.m.mapA < 3 && a.m.Rds &&
                      (D->type == ANIFEM_TENSOR_NULL || D->type == ANIFEM_TENSOR_SCALAR ||
                       D->type == ANIFEM_TENSOR_SYMMETRIC);
     if ((rc = grow<double>(&ctx->d_ebuf, &ctx->ebuf_bytes, piola_row_bytes(S.nf, d0, sym, S.n_tets)))) return rc;
-    *taken = true;
     for (ElemArgs* e : {&a.m, &a.f}) {
         e->coef_n = S.n_tets;
         e->coords = ctx->d_coords;
@@ -1091,7 +1092,8 @@ int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor*
     if (rhs && !a.has_rhs && (rc = fill(rhs, S.ndof, s))) return rc;
     if ((rc = launch_piola(d0, sym, precision == ANIFEM_PREC_FP64, a, static_cast<double*>(ctx->d_ebuf), S.n_tets,
                            (size_t)max_lds, s)))
-        return rc;
+        return rc == ANIFEM_ERR_DIMS ? ANIFEM_OK : rc;  // no LDS left for R beside the context's blocks: not taken
+    *taken = true;
     return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
 }
 

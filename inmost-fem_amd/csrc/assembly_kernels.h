@@ -147,14 +147,15 @@ __device__ __forceinline__ void tri_copy(V* __restrict__ dst, const V* __restric
 //   K_(cb,ca)(b, a) = lam T(cb,b) T(ca,a) + mu (d_{cb,ca} (T^T T)(b,a) + T(ca,b) T(cb,a)),
 // lam and mu scaled by the cell measure.  A compact row holds Tm, lam, mu
 // (kLameCompact values) instead of the 81 values of the nine blocks.
-// The entry of component ca against a reference row r(b, a) needs no block:
+// In FP64 the entry of component ca against a reference row r(b, a) needs no block:
 //   sum_{b,a} K(b, a) r(b, a) = T(ca, .) . z + d_{cb,ca} g,
 //   z_k = lam sum_b T(cb,b) r(b,k) + mu sum_a T(cb,a) r(k,a),  g = mu sum (T^T T) r,
 // z and g shared by the three components: 36 products per reference row in
 // place of 27 and the expansion of the 27 block values, and 21 values held per
-// pair in place of 41.  Every pass forms its entries with these functions,
-// with the roundings fixed (no contraction left to the compiler), so all passes
-// agree bitwise.
+// pair in place of 41.  In FP32 the 27 block values fit the registers, and an
+// entry stays their product with the row, which keeps the values of the FP32
+// mode as they are for the general tensor forms.  Every pass forms its entries
+// with these functions, with the roundings fixed, so all passes agree bitwise.
 constexpr int kLameCompact = 11;
 
 template <typename T>
@@ -162,13 +163,47 @@ struct LameRow {
     T ul[3], um[3];  // lam and mu times row cb of T
     T g[6];          // mu T^T T, packed (sym_pack)
 };
+template <>
+struct LameRow<float> {
+    float k[3][9];  // the blocks (cb, ca)
+};
 
-// c: the compact row; u: row cb of its T (callers read it by address: a runtime
-// index into a register array would move the array to scratch memory).
-template <typename T>
-__device__ __forceinline__ LameRow<T> lame_row(const T* c, const T* u) {
+// u = row cb of T, v = row ca, same = (cb == ca); callers read u and v from
+// the row (or from c with fixed indices): a runtime index into a register
+// array would move the array to scratch memory.
+__device__ __forceinline__ void lame_kblock(const float* c, const float* u, const float* v, bool same, float* Kb) {
 #pragma clang fp contract(off)
-    LameRow<T> L;
+    const float lam = c[9], mu = c[10];
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            float e = lam * (u[b] * v[a]);
+            e = fma(mu, v[b] * u[a], e);
+            const float g = fma(c[b + 6], c[a + 6], fma(c[b + 3], c[a + 3], c[b] * c[a]));
+            const float eg = fma(mu, g, e);
+            Kb[b * 3 + a] = same ? eg : e;
+        }
+}
+
+__device__ __forceinline__ float lame_dot(const float* k, const float* r) {
+    float acc = 0;
+#pragma unroll
+    for (int j = 0; j < 9; ++j) acc = fma(k[j], r[j], acc);
+    return acc;
+}
+
+// c: the compact row; u: row cb of its T.
+__device__ __forceinline__ LameRow<float> lame_row(const float* c, const float* u, int cb) {
+    LameRow<float> L;
+#pragma unroll
+    for (int ca = 0; ca < 3; ++ca) lame_kblock(c, u, c + 3 * ca, cb == ca, L.k[ca]);
+    return L;
+}
+
+__device__ __forceinline__ LameRow<double> lame_row(const double* c, const double* u, int) {
+#pragma clang fp contract(off)
+    LameRow<double> L;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         L.ul[k] = c[9] * u[k];
@@ -181,20 +216,21 @@ __device__ __forceinline__ LameRow<T> lame_row(const T* c, const T* u) {
     return L;
 }
 
-// z and g of one reference row of 9 values.
-template <typename T>
-__device__ __forceinline__ void lame_contract(const LameRow<T>& L, const T* r, T* z, T& g) {
+// What the three components share of one reference row of 9 values: z and g in
+// FP64, nothing in FP32.
+__device__ __forceinline__ void lame_contract(const LameRow<float>&, const float*, float*, float&) {}
+__device__ __forceinline__ void lame_contract(const LameRow<double>& L, const double* r, double* z, double& g) {
 #pragma clang fp contract(off)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        T t = L.ul[0] * r[k];
+        double t = L.ul[0] * r[k];
         t = fma(L.ul[1], r[3 + k], t);
         t = fma(L.ul[2], r[6 + k], t);
         t = fma(L.um[0], r[3 * k], t);
         t = fma(L.um[1], r[3 * k + 1], t);
         z[k] = fma(L.um[2], r[3 * k + 2], t);
     }
-    T t = L.g[0] * r[0];
+    double t = L.g[0] * r[0];
     t = fma(L.g[2], r[4], t);
     t = fma(L.g[5], r[8], t);
     t = fma(L.g[1], r[1] + r[3], t);
@@ -202,18 +238,23 @@ __device__ __forceinline__ void lame_contract(const LameRow<T>& L, const T* r, T
     g = fma(L.g[4], r[5] + r[7], t);
 }
 
-// The entry of the component whose row of T is v; same: it is the pair's own.
-template <typename T>
-__device__ __forceinline__ T lame_value(const T* v, const T* z, T g, bool same) {
+// The entry of component ca (known at compile time), whose row of T is v; same:
+// it is the pair's own.
+__device__ __forceinline__ float lame_value(const LameRow<float>& L, int ca, const float*, const float* r, const float*,
+                                            float, bool) {
+    return lame_dot(L.k[ca], r);
+}
+__device__ __forceinline__ double lame_value(const LameRow<double>&, int, const double* v, const double*, const double* z,
+                                             double g, bool same) {
 #pragma clang fp contract(off)
-    const T e = fma(v[2], z[2], fma(v[1], z[1], v[0] * z[0]));
+    const double e = fma(v[2], z[2], fma(v[1], z[1], v[0] * z[0]));
     return same ? e + g : e;
 }
 
 // The (cb, ca) entry of a compact row in global memory against one reference row.
 template <typename T>
 __device__ __forceinline__ T lame_entry(const T* Kt, int cb, int ca, const T* r) {
-    T c[kLameCompact], u[3], v[3], z[3], g;
+    T c[kLameCompact], u[3], v[3];
 #pragma unroll
     for (int j = 0; j < kLameCompact; ++j) c[j] = Kt[j];
 #pragma unroll
@@ -221,8 +262,16 @@ __device__ __forceinline__ T lame_entry(const T* Kt, int cb, int ca, const T* r)
         u[k] = Kt[3 * cb + k];
         v[k] = Kt[3 * ca + k];
     }
-    lame_contract(lame_row(c, u), r, z, g);
-    return lame_value(v, z, g, cb == ca);
+    if constexpr (sizeof(T) == 4) {
+        T kb[9];
+        lame_kblock(c, u, v, cb == ca, kb);
+        return lame_dot(kb, r);
+    } else {
+        T z[3], g;
+        const LameRow<T> L = lame_row(c, u, cb);
+        lame_contract(L, r, z, g);
+        return lame_value(L, 0, v, r, z, g, cb == ca);
+    }
 }
 
 // Geometry pass over all tets (one lane per tet): FP64 Jacobian, inverse and
@@ -422,7 +471,7 @@ __global__ __launch_bounds__(kBlock) void row_block_kernel(BlockArgs a, const T*
             for (int j = 0; j < kLameCompact; ++j) lc[j] = has_pair ? Kt[j] : T(0);
 #pragma unroll
             for (int k = 0; k < 3; ++k) u[k] = has_pair ? Kt[3 * cb + k] : T(0);
-            lr = lame_row(lc, u);
+            lr = lame_row(lc, u, cb);
         }
     }
     if (qc && !a.lamec) {
@@ -483,9 +532,9 @@ __global__ __launch_bounds__(kBlock) void row_block_kernel(BlockArgs a, const T*
             T acc = 0;
             if (kLame && a.lamec) {
                 if constexpr (kLame) {
-                    T z[3], g;
+                    T z[3], g = 0;
                     lame_contract(lr, Rr, z, g);
-                    acc = lame_value(lc + 3 * ca, z, g, ca == cb);
+                    acc = lame_value(lr, ca, lc + 3 * ca, Rr, z, g, ca == cb);
                 }
             } else if (qc) {
 #pragma unroll
@@ -1110,7 +1159,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
 // every lane works in phase A on a block half as large, and the shorter position
 // lists and slot starts let three waves per SIMD (three workgroups per CU) hide
 // the gathers instead of two.  Same values and sums.  Elasticity on the 48^3
-// cube: pass in FP64 1.69 -> 1.60 ms, in FP32 1.57 -> 1.25; blocks of 102 and 111
+// cube: pass in FP64 1.69 -> 1.56 ms, in FP32 1.57 -> 1.24; blocks of 102 and 111
 // pairs at four waves 1.64 and 1.61, of 256 pairs and one lane 1.77.
 template <int DA0, int DB0, int NC, int NF0, typename T, bool LC = false, bool SPLIT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 1))) void row_block_persistent_vec(BlockArgs a, const T* __restrict__ Kg) {
@@ -1183,10 +1232,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 
         const int cb = (P.ibf & 63) / NF0;
         const T* Kt = Kg + (int64_t)P.tet * a.rowlen;
         if constexpr (LC) {
-#pragma unroll
-            for (int j = 0; j < kLameCompact; ++j) P.c[j] = hp ? Kt[j] : T(0);
+            // u first: its address waits for the pair's component, loaded with the
+            // tet; after the other values its wait would cover those as well
 #pragma unroll
             for (int k = 0; k < 3; ++k) P.u[k] = hp ? Kt[3 * cb + k] : T(0);
+#pragma unroll
+            for (int j = 0; j < kLameCompact; ++j) P.c[j] = hp ? Kt[j] : T(0);
         } else {
 #pragma unroll
             for (int ca = 0; ca < NC; ++ca)
@@ -1246,7 +1297,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 
             const T* Rb = R + ib0 * lenp;
             const int cb = ib / NF0;
             LameRow<T> lr;
-            if constexpr (LC) lr = lame_row(cur.c, cur.u);
+            if constexpr (LC) lr = lame_row(cur.c, cur.u, cb);
             // one reference row per ia0, shared by the NC component entries;
             // columns IA .. IA + HC - 1 (IA = 0, or HC on the second lane of a
             // split pair, whose words start one position early)
@@ -1267,7 +1318,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 
                         if (ps != kPosDropped) {
                             T acc = 0;
                             if constexpr (LC) {
-                                acc = lame_value(cur.c + 3 * ca, z, g, ca == cb);
+                                acc = lame_value(lr, ca, cur.c + 3 * ca, r, z, g, ca == cb);
                             } else {
 #pragma unroll
                                 for (int j = 0; j < KB; ++j) acc += cur.k[ca][j] * r[j];

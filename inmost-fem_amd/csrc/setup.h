@@ -41,8 +41,8 @@ inline BlockCaps default_caps(int nf, bool scalar_space) {
 }
 // Elasticity on three components of P2 (30 entries per pair, the compact Lame
 // rows) takes blocks of 128 pairs as well: two lanes per pair in the fused pass and
-// three workgroups per CU instead of two (48^3 cube: FP64 1.69 -> 1.60 ms, FP32
-// 1.57 -> 1.25).  The scatter of element matrices on these blocks went from 3.37 to
+// three workgroups per CU instead of two (48^3 cube: FP64 1.69 -> 1.56 ms, FP32
+// 1.57 -> 1.24).  The scatter of element matrices on these blocks went from 3.37 to
 // 2.59 ms (FP64 symmetric), 2.94 to 1.89 (FP32 symmetric), 4.41 to 4.08 (FP32
 // general) and 5.51 to 5.67 (FP64 general: whole-row gathers); other tensors, whose
 // pass holds the blocks of K in registers and stays at two workgroups, keep the
