@@ -125,12 +125,15 @@ __global__ void fill_int_kernel(int* p, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
 }
+}  // namespace
+
+namespace anifem {
 // The counts of a pass for the host (one workgroup): the non-finite count, and
 // the degenerate count, summed over the geometry workgroups where each stored
 // its own (deg, n of them).  `host`: pinned words, or null (status only).
-__global__ __launch_bounds__(anifem::kBlock) void publish_counts_kernel(const int* __restrict__ deg, int64_t n, int* status,
+static __global__ __launch_bounds__(kBlock) void publish_counts_kernel(const int* __restrict__ deg, int64_t n, int* status,
                                                                         int* host) {
-    constexpr int B = anifem::kBlock;
+    constexpr int B = kBlock;
     __shared__ int part[B];
     int s = 0;
     if (deg)
@@ -155,13 +158,14 @@ __global__ __launch_bounds__(anifem::kBlock) void publish_counts_kernel(const in
 // The status of the pass queued last on s, counts in d_status (and deg): written
 // by a launch to the thread's pinned words (a copy of 16 bytes from device
 // memory took longer than the small passes it reports on: the 16^3 P1 assembly
-// 38.5 us with it, 30.5 without), or copied where there are none.
+// 38.5 us with it, 30.5 without; the batch of 32 uneven meshes 277 -> 274), or
+// copied where there are none.
 int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, anifem_status* status, hipStream_t s) {
     int* dw = nullptr;
-    volatile int* hw = anifem::host_words(&dw, may_alloc);
+    volatile int* hw = host_words(&dw, may_alloc);
     int h[4] = {0, 0, 0, 0};
     if (hw || deg) {
-        hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(anifem::kBlock), 0, s, deg, n_deg, d_status, dw);
+        hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(kBlock), 0, s, deg, n_deg, d_status, dw);
         ANIFEM_HIP_CHECK(hipGetLastError());
     }
     if (!hw) ANIFEM_HIP_CHECK(hipMemcpyAsync(h, d_status, sizeof(h), hipMemcpyDeviceToHost, s));
@@ -173,6 +177,11 @@ int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, an
     status->reserved = 0;
     return status->code;
 }
+
+}  // namespace anifem
+
+namespace {
+using anifem::read_status;
 
 int fill(double* p, int64_t n, hipStream_t s) {
     if (n <= 0) return ANIFEM_OK;

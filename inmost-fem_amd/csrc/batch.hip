@@ -37,6 +37,7 @@
 #include "setup.h"
 
 namespace anifem {
+int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, anifem_status* status, hipStream_t s);
 int prepare_elem_args(const anifem_op& opA, const anifem_op& opB, const anifem_tensor* D, int order, ElemArgs& a);
 int assembly_create_caps(anifem_assembly** out, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob,
                          const BlockCaps& caps, void* stream, const anifem_vars_desc* vars = nullptr);
@@ -68,10 +69,6 @@ anifem_problem_desc problem_of(int fem, int dirichlet) {
     p.rhs_tensor_storage = ANIFEM_COEF_CONST;
     p.dirichlet = dirichlet;
     return p;
-}
-
-__global__ void batch_status_clear(int* p) {
-    if (threadIdx.x < 4) p[threadIdx.x] = 0;
 }
 
 }  // namespace
@@ -111,6 +108,7 @@ struct anifem_batch {
     int64_t* d_row_ptr = nullptr;  // each mesh's own row_ptr (ndof+1 entries), concatenated
     int32_t* d_col_idx = nullptr;
     int* d_status = nullptr;
+    int* d_deg = nullptr;  // degenerate cells per geometry workgroup
     double* d_K = nullptr;
     // captured launch sequence
     hipStream_t cap_stream = nullptr;
@@ -277,6 +275,7 @@ int capture(anifem_batch* b, const double* kappa, const double* f, double* val, 
     a.val = val;
     a.rhs = rhs;
     a.status = b->d_status;
+    a.deg = b->d_deg;
     a.max_values = b->max_values;
     a.max_pairs = b->max_pairs;
     a.max_slots = b->max_slots;
@@ -351,7 +350,6 @@ int capture(anifem_batch* b, const double* kappa, const double* f, double* val, 
         hipEvent_t e0 = nullptr, e1 = nullptr;
         ANIFEM_HIP_CHECK(hipEventCreate(&e0));
         ANIFEM_HIP_CHECK(hipEventCreate(&e1));
-        hipLaunchKernelGGL(batch_status_clear, dim3(1), dim3(64), 0, rs, b->d_status);
         hipLaunchKernelGGL((geometry_kernel<3, 3, 1, 1, double, true>), dim3((unsigned)gblocks), dim3(kBlock), glds, rs,
                            a, b->d_K, b->n_tets);
         const double* Kt = b->d_K;
@@ -421,7 +419,6 @@ int capture(anifem_batch* b, const double* kappa, const double* f, double* val, 
     b->graph = nullptr;
     hipStream_t s = b->cap_stream;
     ANIFEM_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(batch_status_clear, dim3(1), dim3(64), 0, s, b->d_status);
     hipLaunchKernelGGL((geometry_kernel<3, 3, 1, 1, double, true>), dim3((unsigned)gblocks), dim3(kBlock), glds, s, a,
                        b->d_K, b->n_tets);
     const unsigned grid = (unsigned)(8 * ((b->n_blocks + 7) / 8));
@@ -663,6 +660,8 @@ int anifem_batch_create(anifem_batch** out, int n_meshes, const anifem_batch_mes
     if ((rc = upload_b(p, &p->d_col_idx, col_idx, s))) return rc;
     ANIFEM_HIP_CHECK(hipMalloc((void**)&p->d_status, 4 * sizeof(int)));
     p->bufs.push_back(p->d_status);
+    ANIFEM_HIP_CHECK(hipMalloc((void**)&p->d_deg, (size_t)((p->n_tets + kBlock - 1) / kBlock) * sizeof(int)));
+    p->bufs.push_back(p->d_deg);
     ANIFEM_HIP_CHECK(hipMalloc((void**)&p->d_K, (size_t)p->n_tets * pad16<double>(6 + 1) * sizeof(double)));
     p->bufs.push_back(p->d_K);
     ANIFEM_HIP_CHECK(hipStreamCreateWithFlags(&p->cap_stream, hipStreamNonBlocking));
@@ -751,16 +750,9 @@ int anifem_batch_run(anifem_batch* b, const double* kappa, const double* f, doub
         if (rc) return rc;
     }
     ANIFEM_HIP_CHECK(hipGraphLaunch(b->exec, s));
-    if (status) {
-        int h[4] = {0, 0, 0, 0};
-        ANIFEM_HIP_CHECK(hipMemcpyAsync(h, b->d_status, sizeof(h), hipMemcpyDeviceToHost, s));
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
-        status->n_nonfinite = h[0];
-        status->n_degenerate = h[1];
-        status->code = h[0] ? ANIFEM_ERR_NONFINITE : ANIFEM_OK;
-        status->reserved = 0;
-        return status->code;
-    }
+    if (status)
+        return anifem::read_status(b->d_deg, (b->n_tets + anifem::kBlock - 1) / anifem::kBlock, b->d_status, true,
+                                   status, s);
     return ANIFEM_OK;
 }
 
