@@ -139,8 +139,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 for (int i = 0; i < KB; ++i) Kt[n * KBC + i] = (T)(s * Kb[i]);
             }
         };
-        if (SYM && a.ttype == ANIFEM_TENSOR_SCALAR) {
-            // one T^T T per tet, scaled by the points' coefficients
+        if (SYM && a.ttype == ANIFEM_TENSOR_SCALAR && a.selA <= ANIFEM_GRAD) {
+            // one T^T T per tet, scaled by the points' coefficients (a single
+            // derivative takes part of T only: geometry_block's selector)
             double K1[KB];
             const double* Tm = PIOLA && a.mapA ? JT : PSI;
 #pragma unroll
