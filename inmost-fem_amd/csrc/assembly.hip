@@ -198,6 +198,22 @@ int upload(T** dst, const T* src, size_t count, hipStream_t s) {
     return ANIFEM_OK;
 }
 
+// An array that a call uploads on its first use and a later call, on whatever
+// stream, takes as there: it is resident when the pointer is set.
+template <typename T>
+int upload_resident(T** dst, const T* src, size_t count, hipStream_t s) {
+    if (*dst) return ANIFEM_OK;
+    T* p = nullptr;
+    int rc = upload(&p, src, count, s);
+    if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = ANIFEM_ERR_HIP;
+    if (rc) {
+        if (p) (void)hipFree(p);
+        return rc;
+    }
+    *dst = p;
+    return ANIFEM_OK;
+}
+
 // One colour of the coloured scatter: one lane per (tet of the colour, entry
 // e = ib + nf*ia).  The entry is formed from the tet's geometry row as in the
 // row-block pass and added to its CSR slot; tets of one colour share no node,
@@ -279,10 +295,9 @@ int launch_coloured(anifem_assembly* ctx, const anifem::BlockArgs& a, const T* K
 int upload_maps(anifem_assembly* ctx, hipStream_t s) {
     const anifem::AssemblySetup& S = ctx->S;
     int rc;
-    if (!ctx->d_slot && (rc = upload(&ctx->d_slot, S.slot.data(), S.slot.size(), s))) return rc;
-    if (!ctx->d_dofs && (rc = upload(&ctx->d_dofs, S.dofs.data(), S.dofs.size(), s))) return rc;
-    if (!ctx->d_isdir && (rc = upload(&ctx->d_isdir, S.is_dir.data(), S.is_dir.size(), s))) return rc;
-    return ANIFEM_OK;
+    if ((rc = upload_resident(&ctx->d_slot, S.slot.data(), S.slot.size(), s))) return rc;
+    if ((rc = upload_resident(&ctx->d_dofs, S.dofs.data(), S.dofs.size(), s))) return rc;
+    return upload_resident(&ctx->d_isdir, S.is_dir.data(), S.is_dir.size(), s);
 }
 
 // Persistent row-block pass: occupancy x CUs workgroups, whole XCD groups
@@ -957,8 +972,7 @@ int anifem_assembly_set_scatter(anifem_assembly* ctx, int method) {
         hipStream_t s = nullptr;
         int rc;
         if ((rc = upload_maps(ctx, s))) return rc;
-        if ((rc = upload(&ctx->d_col_tets, ct.data(), ct.size(), s))) return rc;
-        ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
+        if ((rc = upload_resident(&ctx->d_col_tets, ct.data(), ct.size(), s))) return rc;
     }
     ctx->coloured = true;
     return ANIFEM_OK;
@@ -1326,7 +1340,7 @@ int anifem_assembly_eval(anifem_assembly* ctx, int op, const double* xyl, int q,
     const AssemblySetup& S = ctx->S;
     hipStream_t s = static_cast<hipStream_t>(stream);
     int rc;
-    if (!ctx->d_dofs && (rc = upload(&ctx->d_dofs, S.dofs.data(), S.dofs.size(), s))) return rc;
+    if ((rc = upload_resident(&ctx->d_dofs, S.dofs.data(), S.dofs.size(), s))) return rc;
     ApplyArgs a{};
     a.n = S.n_tets;
     a.coords = ctx->d_coords;
@@ -1472,7 +1486,7 @@ int anifem_assembly_run_plain(anifem_assembly* ctx, const anifem_tensor* D, cons
         tab.insert(tab.end(), wq, wq + q);
         tab.insert(tab.end(), v.begin(), v.end());
         tab.insert(tab.end(), wf, wf + qf);
-        if ((rc = upload(&ctx->d_plain_tab, tab.data(), tab.size(), s))) return rc;
+        if ((rc = upload_resident(&ctx->d_plain_tab, tab.data(), tab.size(), s))) return rc;
     }
     if (!ctx->d_plain_tab || !ctx->d_slot || !ctx->d_dofs || !ctx->d_isdir) return ANIFEM_ERR_HIP;
     const double* gtab = ctx->d_plain_tab;
