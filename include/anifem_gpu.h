@@ -150,7 +150,9 @@ int anifem_fem3dface_batch(anifem_op opA, anifem_op opB, const anifem_tensor* D,
  * per-tet DOF values dofs (device, n_tets x nfa: dofs[r*nfa + i]).  opU
  * (device) receives n_tets blocks of dim*q values: opU[r*dim*q + k + dim*n]
  * (for a vector space, component k + 3c of GRAD is du_c/dx_k).  Operators:
- * IDEN and GRAD of P0..P3, CR1, B2, B4; IDEN, DIV and CURL of RT0 and ND0. */
+ * IDEN and GRAD of P0..P3, CR1, B2, B4; IDEN, DIV and CURL of RT0 and ND0.
+ * Returns after enqueueing (xyl is read before that): opU is complete when the
+ * stream has reached the call's end. */
 int anifem_fem3dapply_batch(anifem_op op, const double* xyl, int q, int64_t n_tets, const double* xyz,
                             const double* dofs, double* opU, void* stream);
 /* Batched fem3DapplyX<Op>(XYZ, X, dofs, opU) (eval.h:26-31, eval.inl:103-125):
@@ -441,7 +443,9 @@ int anifem_assembly_run_rhs(anifem_assembly* ctx, const void* F_elem, int elem_p
  * q barycentric points xyl (host, 4q) of each cell, layout as
  * anifem_fem3dapply_batch, caller's cell order.  The cell's DOF values are
  * gathered through the context's DOF map (NATURAL numbering, P3 edge
- * orientation), the step after the solve of examples/tutorials/ex1.cpp:167-168. */
+ * orientation), the step after the solve of examples/tutorials/ex1.cpp:167-168.
+ * Returns after enqueueing, as anifem_fem3dapply_batch; the first evaluation on
+ * a context may upload its DOF map, and waits for that copy. */
 int anifem_assembly_eval(anifem_assembly* ctx, int op, const double* xyl, int q, const double* u, double* opU,
                          void* stream);
 /* Host copy of the tets' node lists after the orientation reorder, caller's

@@ -230,6 +230,15 @@ def _stream_handle(stream):
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
+def _follow(stream):
+    """Order the current stream behind `stream`, if another one was given: its
+    queued work then precedes what the program does with the tensors next."""
+    if stream is not None and _stream_handle(stream) != _stream_handle(None):
+        import torch
+        s = stream if hasattr(stream, "cuda_stream") else torch.cuda.ExternalStream(int(stream))
+        torch.cuda.current_stream().wait_stream(s)
+
+
 # ---- operators (Operator<OP, FemFix<FEM>> / FemVec<n, FEM>) ------------------
 @lru_cache(maxsize=None)
 def _op_sizes(op, fem, ncomp):
@@ -342,7 +351,8 @@ def fem3dface_batch(opA: Op, opB: Op, ttype, storage, D, order, face, xyz, dot_n
 
 def fem3dapply_batch(op: Op, xyl, xyz, dofs, out=None, stream=None):
     """Op(u) at the barycentric points xyl (q, 4) of n tets with per-tet DOF
-    values dofs (device (n, nfa)) (anifem_fem3dapply_batch): (n, q, dim)."""
+    values dofs (device (n, nfa)) (anifem_fem3dapply_batch): (n, q, dim).
+    Queued on `stream`; the current stream is ordered behind it."""
     import torch
     xyl = np.ascontiguousarray(xyl, dtype=np.float64)
     q, n = len(xyl), xyz.shape[1]
@@ -352,6 +362,7 @@ def fem3dapply_batch(op: Op, xyl, xyz, dofs, out=None, stream=None):
         out = torch.empty((n, q, op.dim), dtype=torch.float64, device=xyz.device)
     _check(lib().anifem_fem3dapply_batch(op.c(), _ptr(xyl), q, n, _ptr(xyz), _ptr(dofs), _ptr(out),
                                          _stream_handle(stream)), "anifem_fem3dapply_batch")
+    _follow(stream)
     return out
 
 
@@ -617,7 +628,8 @@ class Assembler:
         """op (IDEN or GRAD; IDEN, DIV or CURL of RT0 / ND0) of the trial
         space's global vector u (device, ndof) at the barycentric points xyl
         (q, 4) of every cell
-        (anifem_assembly_eval): (n_tets, q, dim)."""
+        (anifem_assembly_eval): (n_tets, q, dim).  Queued on `stream`; the
+        current stream is ordered behind it."""
         import torch
         xyl = np.ascontiguousarray(xyl, dtype=np.float64)
         q = len(xyl)
@@ -629,6 +641,7 @@ class Assembler:
             out = torch.empty((self.n_tets, q, dim), dtype=torch.float64, device=u.device)
         _check(lib().anifem_assembly_eval(self._h, op, _ptr(xyl), q, _ptr(u), _ptr(out), _stream_handle(stream)),
                "anifem_assembly_eval")
+        _follow(stream)
         return out
 
     def quadrature_points(self, order=None, out=None, stream=None):

@@ -35,3 +35,28 @@ def test_first_use_of_the_dof_map_is_complete_for_other_streams(first):
     other.synchronize()
     for o in outs:
         assert torch.equal(o, expected)
+
+
+@pytest.mark.parametrize("handle", [False, True])
+@pytest.mark.parametrize("call", ["evaluate", "apply"])
+def test_result_of_another_stream_is_read_in_order(call, handle):
+    """The current stream follows the stream that was given to the call: reading
+    the result at once gives the values, with the given stream still busy."""
+    import torch
+    coords, tets = af.kuhn_cube(5, 0.2, 7)
+    xyl = np.random.default_rng(8).dirichlet(np.ones(4), 3)
+    op = af.Op(af.GRAD, af.FEM_P2)
+    asm = af.Assembler(coords, tets, op, dirichlet=af.DIRICHLET_BOUNDARY)
+    u = torch.from_numpy(np.random.default_rng(9).normal(size=asm.ndof)).cuda()
+    dofs = torch.from_numpy(np.random.default_rng(9).normal(size=(len(tets), op.nfa))).cuda()
+    xyz = torch.from_numpy(np.ascontiguousarray(coords[tets].reshape(len(tets), 12).T)).cuda()
+    run = {"evaluate": lambda **k: asm.evaluate(u, xyl, **k),
+           "apply": lambda **k: af.fem3dapply_batch(op, xyl, xyz, dofs, **k)}[call]
+    expected = run().cpu()
+    out = torch.full(expected.shape, np.nan, dtype=torch.float64, device="cuda")
+    busy = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(20_000_000)
+    got = run(out=out, stream=busy.cuda_stream if handle else busy).cpu()
+    assert torch.equal(got, expected)
