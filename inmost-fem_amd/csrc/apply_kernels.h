@@ -34,11 +34,34 @@ __host__ __device__ constexpr int apply_nf0(int fem) {
 // wave write different banks.
 __host__ __device__ inline int apply_stage_row(int pc, int dim) { return (pc * dim) | 1; }
 
-// Points per pass: the staged values of a workgroup stay within 32 KB.
-inline int apply_chunk(int q, int dim) {
-    int pc = q;
-    while (pc > 1 && (size_t)kBlock * apply_stage_row(pc, dim) * sizeof(double) > 32 * 1024) --pc;
-    return pc;
+// Workgroups that a launch has room for (four per CU).
+constexpr int64_t kApplyGroups = 1024;
+
+// Points per pass, by the stage's share of the LDS.  32 KB keeps five workgroups
+// on a CU; 60 KB where even so there are more than kApplyGroups passes to make:
+// each then reads the cells' DOFs for more points and stores longer ranges (GRAD
+// of P3^3 at 14 points, 20,001 cells: 38 us with 32 KB, 19 with 60; of 3,001 cells
+// 8.0 and 11.5).
+inline int apply_chunk(int64_t n, int q, int dim) {
+    auto fit = [&](size_t bytes) {
+        int pc = q;
+        while (pc > 1 && (size_t)kBlock * apply_stage_row(pc, dim) * sizeof(double) > bytes) --pc;
+        return pc;
+    };
+    const int64_t cells = (n + kBlock - 1) / kBlock;
+    const int pc = fit(32 * 1024);
+    return cells * ((q + pc - 1) / pc) > kApplyGroups ? fit(60 * 1024) : pc;
+}
+
+// Workgroups along the passes of a cell range (blockIdx.y), each with its own
+// run of points.  Cells that fill the chip by themselves take one, which reads
+// their DOFs once; fewer leave it to a chain of up to q passes in few workgroups
+// (GRAD of P3^3 at 96 points: 255 cells 384 us against 7.7, 3,001 cells 387
+// against 16; one lane per (cell, point) took 58 and 114).
+inline int apply_split(int64_t n, int q, int pc) {
+    const int64_t cells = (n + kBlock - 1) / kBlock, passes = (q + pc - 1) / pc;
+    const int64_t want = (kApplyGroups + cells - 1) / cells;
+    return (int)(want < passes ? want : passes);
 }
 
 // D: reference components per basis function (ApplyArgs::d).
@@ -64,8 +87,10 @@ __global__ __launch_bounds__(kBlock) void apply_points_kernel(ApplyArgs a, Apply
         tet_geometry(P, PSI, det);
         tet_jacobian_t(P, JT);
     }
-    for (int p0 = 0; p0 < a.q; p0 += pc) {
-        const int np = a.q - p0 < pc ? a.q - p0 : pc;
+    const int share = ((a.q + pc - 1) / pc + gridDim.y - 1) / gridDim.y * pc;  // points of this workgroup
+    const int p_end = min(a.q, (int)(blockIdx.y + 1) * share);
+    for (int p0 = blockIdx.y * share; p0 < p_end; p0 += pc) {
+        const int np = p_end - p0 < pc ? p_end - p0 : pc;
         if ((int)threadIdx.x < np) {
             double L[4], u[NF0 * D];
 #pragma unroll
@@ -135,7 +160,7 @@ __global__ __launch_bounds__(kBlock) void apply_points_kernel(ApplyArgs a, Apply
                 ++cell;
             }
         }
-        if (p0 + pc < a.q) __syncthreads();  // table and stage are rewritten
+        if (p0 + pc < p_end) __syncthreads();  // table and stage are rewritten
     }
 }
 

@@ -329,9 +329,9 @@ static int prepare_apply(const anifem_op& op, int q, ApplyArgs& a) {
 
 template <int FEM, int D>
 static int launch_points(const ApplyArgs& a, const ApplyPoints& pts, bool mesh, hipStream_t s) {
-    const int dim = a.map >= 3 ? 9 : D * a.ncomp, pc = apply_chunk(a.q, dim);
+    const int dim = a.map >= 3 ? 9 : D * a.ncomp, pc = apply_chunk(a.n, a.q, dim);
     const size_t lds = ((size_t)pc * apply_nf0(FEM) * D + (size_t)kBlock * apply_stage_row(pc, dim)) * sizeof(double);
-    const dim3 grid((unsigned)((a.n + kBlock - 1) / kBlock));
+    const dim3 grid((unsigned)((a.n + kBlock - 1) / kBlock), (unsigned)apply_split(a.n, a.q, pc));
     if (mesh) hipLaunchKernelGGL((apply_points_kernel<FEM, D, true>), grid, dim3(kBlock), lds, s, a, pts, pc);
     else hipLaunchKernelGGL((apply_points_kernel<FEM, D, false>), grid, dim3(kBlock), lds, s, a, pts, pc);
     ANIFEM_HIP_CHECK(hipGetLastError());
