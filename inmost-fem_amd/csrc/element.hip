@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -338,6 +339,26 @@ static int launch_points(const ApplyArgs& a, const ApplyPoints& pts, bool mesh, 
     return ANIFEM_OK;
 }
 
+// f(space, reference components) with both as compile-time constants.
+template <typename F>
+static int for_space(int fem, int d, F f) {
+    auto with = [&](auto space) {
+        return d == 3 ? f(space, std::integral_constant<int, 3>{}) : f(space, std::integral_constant<int, 1>{});
+    };
+    switch (fem) {
+        case ANIFEM_FEM_P0: return with(std::integral_constant<int, ANIFEM_FEM_P0>{});
+        case ANIFEM_FEM_P1: return with(std::integral_constant<int, ANIFEM_FEM_P1>{});
+        case ANIFEM_FEM_P2: return with(std::integral_constant<int, ANIFEM_FEM_P2>{});
+        case ANIFEM_FEM_P3: return with(std::integral_constant<int, ANIFEM_FEM_P3>{});
+        case ANIFEM_FEM_CR1: return with(std::integral_constant<int, ANIFEM_FEM_CR1>{});
+        case ANIFEM_FEM_B2: return with(std::integral_constant<int, ANIFEM_FEM_B2>{});
+        case ANIFEM_FEM_B4: return with(std::integral_constant<int, ANIFEM_FEM_B4>{});
+        case ANIFEM_FEM_RT0: return with(std::integral_constant<int, ANIFEM_FEM_RT0>{});
+        case ANIFEM_FEM_ND0: return with(std::integral_constant<int, ANIFEM_FEM_ND0>{});
+    }
+    return ANIFEM_ERR_ARG;
+}
+
 // op at q barycentric points xyl (host) common to all cells.
 int launch_apply(const anifem_op& op, const double* xyl, int q, ApplyArgs a, bool mesh, hipStream_t s) {
     if (!xyl) return ANIFEM_ERR_ARG;
@@ -346,27 +367,17 @@ int launch_apply(const anifem_op& op, const double* xyl, int q, ApplyArgs a, boo
     if (a.n == 0) return ANIFEM_OK;
     ApplyPoints pts;
     std::copy(xyl, xyl + 4 * q, pts.xyl);
-    switch (op.fem) {
-        case ANIFEM_FEM_P0:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_P0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P0, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_P1:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_P1, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P1, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_P2:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_P2, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P2, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_P3:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_P3, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_P3, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_CR1:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_CR1, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_CR1, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_B2:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_B2, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_B2, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_B4:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_B4, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_B4, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_RT0:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_RT0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_RT0, 1>(a, pts, mesh, s);
-        case ANIFEM_FEM_ND0:
-            return a.d == 3 ? launch_points<ANIFEM_FEM_ND0, 3>(a, pts, mesh, s) : launch_points<ANIFEM_FEM_ND0, 1>(a, pts, mesh, s);
-    }
-    return ANIFEM_ERR_ARG;
+    return for_space(op.fem, a.d, [&](auto fem, auto d) { return launch_points<fem.value, d.value>(a, pts, mesh, s); });
+}
+
+// op at each cell's own physical points.
+static int launch_apply_x(const anifem_op& op, const ApplyArgs& a, hipStream_t s) {
+    return for_space(op.fem, a.d, [&](auto fem, auto d) {
+        const int64_t blocks = (a.n * a.q + kBlock - 1) / kBlock;
+        hipLaunchKernelGGL((apply_x_kernel<fem.value, d.value>), dim3((unsigned)blocks), dim3(kBlock), 0, s, a);
+        ANIFEM_HIP_CHECK(hipGetLastError());
+        return ANIFEM_OK;
+    });
 }
 }  // namespace anifem
 
@@ -383,10 +394,7 @@ extern "C" int anifem_fem3dapplyx_batch(anifem_op op, int q, int64_t n_tets, con
     a.X = X;
     a.dofs = dofs;
     a.out = opU;
-    const int64_t blocks = (a.n * a.q + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(apply_x_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
-    ANIFEM_HIP_CHECK(hipGetLastError());
-    return ANIFEM_OK;
+    return launch_apply_x(op, a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int anifem_fem3dapply_batch(anifem_op op, const double* xyl, int q, int64_t n_tets, const double* xyz,

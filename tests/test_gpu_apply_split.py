@@ -35,3 +35,29 @@ def test_split_points_match_oracle(op, fem, nc, q, n):
     scale = np.abs(ref).max(axis=(1, 2), keepdims=True)
     assert (np.abs(got - ref) <= 1e-12 * scale).all()
     assert torch.equal(out, out[:m][torch.from_numpy(cell).cuda()])
+
+
+@pytest.mark.parametrize("fem", [af.FEM_P0, af.FEM_P1, af.FEM_P2, af.FEM_P3, af.FEM_CR1, af.FEM_B2, af.FEM_B4,
+                                 af.FEM_RT0, af.FEM_ND0])
+def test_points_of_each_cell_match_oracle(fem):
+    """Every space and operator at each cell's own physical points
+    (anifem_fem3dapplyx_batch): the cells of a mesh, whose barycentric coordinates
+    lose no digits; <= 1e-12 of the largest value."""
+    import torch
+    vector = fem in (af.FEM_RT0, af.FEM_ND0)
+    coords, tets = af.kuhn_cube(3, 0.2, 11)
+    n, q = 129, 3
+    xyz = coords[tets[:n]].reshape(n, 12)
+    rng = np.random.default_rng(fem)
+    X = T.points_physical(xyz, rng.dirichlet(np.ones(4), q))
+    for op, nc in [(af.IDEN, 1), (af.GRAD, 1)] + ([(af.DIV, 1), (af.CURL, 1)] if vector else
+                                                  [(af.IDEN, 2), (af.IDEN, 3), (af.GRAD, 2), (af.GRAD, 3)]):
+        o = af.Op(op, fem, nc)
+        dofs = rng.normal(size=(n, o.nfa))
+        got = af.fem3dapplyx_batch(o, torch.from_numpy(X).cuda(), torch.from_numpy(T.soa_xyz(xyz)).cuda(),
+                                   torch.from_numpy(dofs).cuda()).cpu().numpy()
+        if fem == af.FEM_P0 and op == af.GRAD:  # zero; the oracle has values of P0 only
+            ref = np.zeros((n, q, o.dim))
+        else:
+            ref = T.orc_applyx(op, fem, nc, X, xyz, dofs)
+        assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max(), (op, nc)
