@@ -48,6 +48,24 @@ void reference_tensor(int opA, int femA, int opB, int femB, int order, bool per_
 int triangle_quadrature(int order, const double** p, const double** w);
 int rule_points(int order, int face, std::vector<double>& pts, std::vector<double>& wts);
 
+// The per-point reference tensor in the B-operand order of the 16x16x4 matrix
+// instructions: f[(et*ks + k)*64 + l] = R[entry 16 et + l % 16][kk =
+// 4 k + l / 16], kk over q KB values, zero beyond the table; ks, the instructions
+// along kk, is a multiple of four (the kernel's unrolling).  Entry u is ib + 256 ia = ent[u] (kNoEntry
+// past n_ent): every entry, column by column, or with `packed` (a symmetric K of
+// 6 values per point: columns of K(a, b) and K(b, a) summed) those with ib >= ia.
+constexpr int kNoEntry = 0xFFFF;
+struct RefFragDev {
+    const double* f64 = nullptr;
+    const float* f32 = nullptr;
+    const uint16_t* ent = nullptr;
+    int ks = 0, n_ent = 0;
+};
+inline int frag_steps(int q, int kbc) { return (q * kbc + 15) / 16 * 4; }
+// K of 16 tets for ks instructions, padded as the per-point kernel pads it, is
+// within the LDS it may use.
+inline bool frag_fits(int ks, int elem_bytes) { return (size_t)16 * 4 * (ks + 1) * elem_bytes <= 64 * 1024; }
+
 // Device-resident copies of reference tensors, built lazily per (pair, order,
 // per_point) and kept for the life of the process.
 struct RefTensorDev {
@@ -71,27 +89,17 @@ struct RefTensorDev {
     // rs64 row (ib + nfB ia) equals row (ia + nfB ib) bit for bit (one space
     // and one operator on both sides; checked when the table is built)
     bool rs_sym = false;
+    // per-point tensors (more than one point): the table in operand order, and
+    // packed where one 3-dimensional operator stands on both sides; null where
+    // frag_fits does not hold in FP32.  Built with the table and not when a call
+    // first needs them: a call whose table is there allocates nothing, so that
+    // it can be captured.
+    RefFragDev frag, frag_sym;
 };
 // Packed index of K(a, b) = K(b, a) in the symmetric layout above.
 __host__ __device__ inline int sym_pack(int a, int b) { return a <= b ? a + b * (b + 1) / 2 : b + a * (a + 1) / 2; }
 int get_ref_tensor(int opA, int femA, int opB, int femB, int order, bool per_point, RefTensorDev* out,
                    int face = -1);
-// The per-point reference tensor in the B-operand order of the 16x16x4 matrix
-// instructions: f[(et*ks + k)*64 + l] = R[entry 16 et + l % 16][kk =
-// 4 k + l / 16], kk over q KB values, zero beyond the table; ks, the instructions
-// along kk, is a multiple of four (the kernel's unrolling).  Entry u is ib + 256 ia = ent[u] (kNoEntry
-// past n_ent): every entry, column by column, or with `packed` (a symmetric K of
-// 6 values per point: columns of K(a, b) and K(b, a) summed) those with ib >= ia.
-// Built lazily and kept like the tensors above.
-constexpr int kNoEntry = 0xFFFF;
-struct RefFragDev {
-    const double* f64 = nullptr;
-    const float* f32 = nullptr;
-    const uint16_t* ent = nullptr;
-    int ks = 0, n_ent = 0;
-};
-inline int frag_steps(int q, int kbc) { return (q * kbc + 15) / 16 * 4; }
-int get_ref_fragments(int opA, int femA, int opB, int femB, int order, int face, bool packed, RefFragDev* out);
 // Set by entry points that must not allocate device memory: get_ref_tensor
 // then only looks tables up and fails with ANIFEM_ERR_ARG where one would
 // have to be built.

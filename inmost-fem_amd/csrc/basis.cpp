@@ -360,6 +360,41 @@ __global__ void split_f16_kernel(const float* x, int64_t n, _Float16* out) {
 
 thread_local bool g_ref_lookup_only = false;
 
+// The operand-order table of R (per point, q points).
+static int build_fragments(const std::vector<double>& R, int nfA, int nfB, int KB, int q, bool packed, RefFragDev* out) {
+    const int KBC = packed ? 6 : KB;
+    std::vector<uint16_t> ent;
+    for (int ia = 0; ia < nfA; ++ia)
+        for (int ib = packed ? ia : 0; ib < nfB; ++ib) ent.push_back((uint16_t)(ib + 256 * ia));
+    RefFragDev t;
+    t.n_ent = (int)ent.size();
+    t.ks = frag_steps(q, KBC);
+    if (!frag_fits(t.ks, 4)) return ANIFEM_OK;
+    const size_t nt = (ent.size() + 15) / 16, steps = t.ks;
+    std::vector<double> f(nt * steps * 64, 0.0);
+    for (size_t u = 0; u < ent.size(); ++u)
+        for (int n = 0; n < q; ++n)
+            for (int c = 0; c < KB; ++c) {
+                const int rr = (ent[u] & 0xFF) + nfB * (ent[u] >> 8);
+                const int kk = n * KBC + (packed ? sym_pack(c / 3, c % 3) : c);
+                f[((u / 16) * steps + kk / 4) * 64 + u % 16 + 16 * (kk % 4)] += R[((size_t)rr * q + n) * KB + c];
+            }
+    ent.resize(nt * 16, (uint16_t)kNoEntry);
+    const std::vector<float> ff(f.begin(), f.end());
+    void *d64 = nullptr, *d32 = nullptr, *de = nullptr;
+    ANIFEM_HIP_CHECK(hipMalloc(&d64, f.size() * sizeof(double)));
+    ANIFEM_HIP_CHECK(hipMalloc(&d32, f.size() * sizeof(float)));
+    ANIFEM_HIP_CHECK(hipMalloc(&de, ent.size() * sizeof(uint16_t)));
+    ANIFEM_HIP_CHECK(hipMemcpy(d64, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice));
+    ANIFEM_HIP_CHECK(hipMemcpy(d32, ff.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
+    ANIFEM_HIP_CHECK(hipMemcpy(de, ent.data(), ent.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+    t.f64 = static_cast<const double*>(d64);
+    t.f32 = static_cast<const float*>(d32);
+    t.ent = static_cast<const uint16_t*>(de);
+    *out = t;
+    return ANIFEM_OK;
+}
+
 int get_ref_tensor(int opA, int femA, int opB, int femB, int order, bool per_point, RefTensorDev* out, int face) {
     static std::mutex mu;
     static std::map<std::tuple<int, int, int, int, int, int, int, int>, RefTensorDev> cache;
@@ -395,6 +430,13 @@ int get_ref_tensor(int opA, int femA, int opB, int femB, int order, bool per_poi
     ANIFEM_HIP_CHECK(hipMemcpy(d32, Rf.data(), Rf.size() * sizeof(float), hipMemcpyHostToDevice));
     t.r64 = static_cast<const double*>(d64);
     t.r32 = static_cast<const float*>(d32);
+    if (per_point && t.q > 1) {
+        const int nA = nf_scalar(femA), nB = nf_scalar(femB);
+        int rc = build_fragments(R, nA, nB, t.KB, t.q, false, &t.frag);
+        if (!rc && t.KB == 9 && opA == opB && femA == femB)
+            rc = build_fragments(R, nA, nB, t.KB, t.q, true, &t.frag_sym);
+        if (rc) return rc;
+    }
     if (!per_point && t.KB == 9) {
         // columns kk = b*3 + a of K(b, a), summed onto the packed K(a, b)
         std::vector<double> Rs((size_t)t.E0 * 6, 0.0);
@@ -441,54 +483,6 @@ int get_ref_tensor(int opA, int femA, int opB, int femB, int order, bool per_poi
         ANIFEM_HIP_CHECK(hipFree(dx));
         t.r16 = d16;
     }
-    cache[key] = t;
-    *out = t;
-    return ANIFEM_OK;
-}
-
-int get_ref_fragments(int opA, int femA, int opB, int femB, int order, int face, bool packed, RefFragDev* out) {
-    static std::mutex mu;
-    static std::map<std::tuple<int, int, int, int, int, int, int, int>, RefFragDev> cache;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return ANIFEM_ERR_HIP;
-    const auto key = std::make_tuple(dev, opA, femA, opB, femB, order, face, (int)packed);
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) {
-        *out = it->second;
-        return ANIFEM_OK;
-    }
-    std::vector<double> R;
-    reference_tensor(opA, femA, opB, femB, order, true, R, face);
-    const int nfA = nf_scalar(femA), nfB = nf_scalar(femB), KB = ref_dim(opA, femA) * ref_dim(opB, femB);
-    const int q = (int)(R.size() / ((size_t)nfA * nfB * KB)), KBC = packed ? 6 : KB;
-    std::vector<uint16_t> ent;
-    for (int ia = 0; ia < nfA; ++ia)
-        for (int ib = packed ? ia : 0; ib < nfB; ++ib) ent.push_back((uint16_t)(ib + 256 * ia));
-    RefFragDev t;
-    t.n_ent = (int)ent.size();
-    t.ks = frag_steps(q, KBC);
-    const size_t nt = (ent.size() + 15) / 16, steps = t.ks;
-    std::vector<double> f(nt * steps * 64, 0.0);
-    for (size_t u = 0; u < ent.size(); ++u)
-        for (int n = 0; n < q; ++n)
-            for (int c = 0; c < KB; ++c) {
-                const int rr = (ent[u] & 0xFF) + nfB * (ent[u] >> 8);
-                const int kk = n * KBC + (packed ? sym_pack(c / 3, c % 3) : c);
-                f[((u / 16) * steps + kk / 4) * 64 + u % 16 + 16 * (kk % 4)] += R[((size_t)rr * q + n) * KB + c];
-            }
-    ent.resize(nt * 16, (uint16_t)kNoEntry);
-    const std::vector<float> ff(f.begin(), f.end());
-    void *d64 = nullptr, *d32 = nullptr, *de = nullptr;
-    ANIFEM_HIP_CHECK(hipMalloc(&d64, f.size() * sizeof(double)));
-    ANIFEM_HIP_CHECK(hipMalloc(&d32, f.size() * sizeof(float)));
-    ANIFEM_HIP_CHECK(hipMalloc(&de, ent.size() * sizeof(uint16_t)));
-    ANIFEM_HIP_CHECK(hipMemcpy(d64, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice));
-    ANIFEM_HIP_CHECK(hipMemcpy(d32, ff.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
-    ANIFEM_HIP_CHECK(hipMemcpy(de, ent.data(), ent.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
-    t.f64 = static_cast<const double*>(d64);
-    t.f32 = static_cast<const float*>(d32);
-    t.ent = static_cast<const uint16_t*>(de);
     cache[key] = t;
     *out = t;
     return ANIFEM_OK;

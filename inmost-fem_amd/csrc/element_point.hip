@@ -82,11 +82,11 @@ int launch_element_point(const anifem_op& opA, const anifem_op& opB, int order, 
     const int kstride = opA.ncomp * opB.ncomp * a.q * dA * dB, es = fp64 ? 8 : 4;
     const int ns = (a.scA | a.scB) ? a.nfA0 + a.nfB0 : 0;
     if (element_scale_offset(4, kstride, es) + 4 * ns * sizeof(double) > 64 * 1024) return ANIFEM_OK;
-    // the table of a rule whose K cannot fit is not built
-    if ((size_t)16 * point_stride(frag_steps(a.q, sym ? 6 : dA * dB)) * es > 64 * 1024) return ANIFEM_OK;
-    RefFragDev f;
-    const int rc = get_ref_fragments(opA.op, opA.fem, opB.op, opB.fem, order, a.face, sym, &f);
+    if (!frag_fits(frag_steps(a.q, sym ? 6 : dA * dB), es)) return ANIFEM_OK;
+    RefTensorDev R;  // as prepared for the call: the table is there
+    const int rc = get_ref_tensor(opA.op, opA.fem, opB.op, opB.fem, order, true, &R, a.face);
     if (rc) return rc;
+    const RefFragDev& f = sym ? R.frag_sym : R.frag;
     a.frag = fp64 ? static_cast<const void*>(f.f64) : static_cast<const void*>(f.f32);
     a.ent = f.ent;
     a.ks = f.ks;
