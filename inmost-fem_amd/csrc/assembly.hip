@@ -24,7 +24,7 @@ int prepare_elem_args(const anifem_op& opA, const anifem_op& opB, const anifem_t
 int launch_physical_points(int order, int64_t n, const double* xyz, const double* coords, const int32_t* tetnodes,
                            int64_t nodes_stride, double* X, hipStream_t s);
 int launch_apply(const anifem_op& op, const double* xyl, int q, ApplyArgs a, bool mesh, hipStream_t s);
-size_t piola_row_bytes(int nf, int d0, bool sym, int64_t n);
+size_t piola_row_bytes(int nf, int d0, int64_t n);
 int launch_piola(int d0, bool sym, bool fp64, const BlockArgs& a, double* rows, int64_t n, size_t max_lds,
                  hipStream_t s);
 }  // namespace anifem
@@ -1096,7 +1096,7 @@ int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor*
     const bool sym = precision == ANIFEM_PREC_FP64 && d0 == 3 && a.m.mapA < 3 && a.m.Rds &&
                      (D->type == ANIFEM_TENSOR_NULL || D->type == ANIFEM_TENSOR_SCALAR ||
                       D->type == ANIFEM_TENSOR_SYMMETRIC);
-    if ((rc = grow<double>(&ctx->d_ebuf, &ctx->ebuf_bytes, piola_row_bytes(S.nf, d0, sym, S.n_tets)))) return rc;
+    if ((rc = grow<double>(&ctx->d_ebuf, &ctx->ebuf_bytes, piola_row_bytes(S.nf, d0, S.n_tets)))) return rc;
     for (ElemArgs* e : {&a.m, &a.f}) {
         e->coef_n = S.n_tets;
         e->coords = ctx->d_coords;

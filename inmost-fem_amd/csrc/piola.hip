@@ -31,9 +31,11 @@ int launch_dim(int d0, bool sym, const BlockArgs& a, double* rows, int64_t n, si
 
 }  // namespace
 
-// Bytes of the cells' rows for nf local DOFs of a d0-component reference field.
-size_t piola_row_bytes(int nf, int d0, bool sym, int64_t n) {
-    return (size_t)n * piola_rowlen(nf, d0 == 1 ? 1 : (sym ? 6 : 9)) * sizeof(double);
+// Bytes of the cells' rows for nf local DOFs of a d0-component reference field, in
+// the longest form (K not packed): a pass in the other precision, whose rows may
+// be longer, then finds room without another allocation.
+size_t piola_row_bytes(int nf, int d0, int64_t n) {
+    return (size_t)n * piola_rowlen(nf, d0 == 1 ? 1 : 9) * sizeof(double);
 }
 
 int launch_piola(int d0, bool sym, bool fp64, const BlockArgs& a, double* rows, int64_t n, size_t max_lds,
