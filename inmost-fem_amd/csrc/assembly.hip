@@ -1104,8 +1104,7 @@ int run_piola(anifem_assembly* ctx, const anifem_tensor* D, const anifem_tensor*
         e->nodes_stride = S.n_tets;
     }
     a.n_kinds = 1;
-    a.kinds[0] = KindTable{sym ? a.m.Rds : a.m.Rd, sym ? a.m.Rfs : a.m.Rf, nullptr, nullptr, a.m.nfA0, a.m.nfB0, S.nf,
-                           S.nf * S.nf, 0, 0};
+    a.kinds[0] = KindTable{sym ? a.m.Rds : a.m.Rd, a.m.Rf, nullptr, nullptr, a.m.nfA0, a.m.nfB0, S.nf, S.nf * S.nf, 0, 0};
     set_block_lists(ctx, a);
     a.val = csr_val;
     a.rhs = rhs;

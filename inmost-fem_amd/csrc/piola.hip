@@ -23,10 +23,14 @@ int launch(const BlockArgs& a, double* rows, int64_t n, size_t max_lds, hipStrea
     return ANIFEM_OK;
 }
 
+// sym: K packed, in FP64 only.
 template <int NF, typename T>
 int launch_dim(int d0, bool sym, const BlockArgs& a, double* rows, int64_t n, size_t max_lds, hipStream_t s) {
     if (d0 == 1) return launch<1, 1, NF, T>(a, rows, n, max_lds, s);
-    return sym ? launch<3, 6, NF, T>(a, rows, n, max_lds, s) : launch<3, 9, NF, T>(a, rows, n, max_lds, s);
+    if constexpr (sizeof(T) == 8) {
+        if (sym) return launch<3, 6, NF, T>(a, rows, n, max_lds, s);
+    }
+    return launch<3, 9, NF, T>(a, rows, n, max_lds, s);
 }
 
 }  // namespace
