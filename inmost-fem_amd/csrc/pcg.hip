@@ -725,7 +725,6 @@ constexpr int kSmallRows = 5 * kSmallThreads;
 constexpr int kSmallChunk = 8;                // entries of a row per load group
 constexpr int kSmallChunks = 192;             // load groups of 64 rows, in all
 constexpr int64_t kSmallNnz = 48 * 1024;
-constexpr int kNotTaken = 2;                   // PcgState::done: the rows do not fit the slots
 
 // One step of a wave sum: the value CTRL lanes away (data-parallel primitive),
 // zero where there is none or the row is masked out.
@@ -771,6 +770,32 @@ __device__ __forceinline__ void small_sums(double (&v)[NV], double (*sh)[kSmallW
     }
 }
 
+// Load groups of the slice of 64 rows at `base`, in every lane of the wave.
+__device__ __forceinline__ int64_t slice_groups(int64_t base, int n, const int64_t* rp) {
+    const int64_t row = base + threadIdx.x % 64;
+    int64_t m = row < n ? rp[row + 1] - rp[row] : 0;
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (int64_t)__shfl_xor((long long)m, o, 64));
+    return (m + kSmallChunk - 1) / kSmallChunk;
+}
+
+// What the host has to know of a system of at most kSmallRows rows (one
+// workgroup): its entries, and the load groups that its padded layout takes.
+__global__ __launch_bounds__(kSmallThreads) void small_size_kernel(int n, const int64_t* __restrict__ rp, int64_t* host) {
+    __shared__ int64_t part[kSmallWaves];
+    const int w = threadIdx.x / 64;
+    int64_t groups = 0;
+    for (int64_t base = 64 * w; base < n; base += 64 * kSmallWaves) groups += slice_groups(base, n, rp);
+    if (threadIdx.x % 64 == 0) part[w] = groups;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kSmallWaves; ++i) groups += part[i];
+        host[0] = rp[n];
+        host[1] = groups;
+        __threadfence_system();
+    }
+}
+
+// The system's layout takes at most kSmallChunks load groups (small_size_kernel).
 template <int R>
 __global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const int64_t* __restrict__ rp,
                                                                    const int32_t* __restrict__ ci,
@@ -789,20 +814,15 @@ __global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const i
     for (int i = 0; i < R; ++i) {
         const int row = 64 * (w + kSmallWaves * i) + l;
         q0[i] = row < n ? rp[row] : 0;
-        len[i] = row < n ? (int)min(rp[row + 1] - q0[i], (int64_t)kSmallChunk * (kSmallChunks + 1)) : 0;
-        int m = len[i];
-        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
-        if (l == 0) off[w * R + i + 1] = (m + kSmallChunk - 1) / kSmallChunk;
+        len[i] = row < n ? (int)(rp[row + 1] - q0[i]) : 0;
+        const int m = (int)slice_groups(64 * (w + kSmallWaves * i), n, rp);
+        if (l == 0) off[w * R + i + 1] = m;
     }
     if (threadIdx.x == 0) off[0] = 0;
     __syncthreads();
     if (threadIdx.x == 0)
         for (int s = 0; s < kSmallWaves * R; ++s) off[s + 1] += off[s];
     __syncthreads();
-    if (off[kSmallWaves * R] > kSmallChunks) {  // uniform
-        if (threadIdx.x == 0) st->done = kNotTaken;
-        return;
-    }
     double xr[R], rr_[R], di[R], ap[R];
     int g1[R];
     double s3[3] = {0.0, 0.0, 0.0};  // r.z, r.r, b.b
@@ -1234,8 +1254,29 @@ int workspace(int slot, size_t bytes, void** out) {
 // Systems the one-workgroup solver takes: rows within its LDS and registers
 // and a matrix that streams faster than two launches run: 46,941 entries of 16^3
 // P1 8.7 against 13.2 us an iteration, 51,109 of P2 at 7^3 (rows of 10 to 65, wider
-// slices) 14.9 against 14.7; at 4,437 entries 3.9 against 15.7.
-bool small_system(int64_t n, int64_t nnz) { return n <= kSmallRows && nnz <= kSmallNnz; }
+// slices) 14.9 against 14.7; at 4,437 entries 3.9 against 15.7.  Both sizes come
+// from row_ptr before anything else is queued.
+bool small_system(int64_t n, int64_t nnz, int64_t groups) {
+    return n <= kSmallRows && nnz <= kSmallNnz && groups <= kSmallChunks;
+}
+
+// The entries of the matrix, and for a system that may be small the load groups
+// of its layout (-1 where the host words to pass them are missing).  Waits for s.
+int system_size(int64_t n, const int64_t* rp, int64_t* nnz, int64_t* groups, hipStream_t s) {
+    int* dw = nullptr;
+    volatile int64_t* hw = n <= kSmallRows ? reinterpret_cast<volatile int64_t*>(host_words(&dw, true)) : nullptr;
+    *groups = -1;
+    if (hw) {
+        hipLaunchKernelGGL(small_size_kernel, dim3(1), dim3(kSmallThreads), 0, s, (int)n, rp,
+                           reinterpret_cast<int64_t*>(dw));
+        ANIFEM_HIP_CHECK(hipGetLastError());
+    } else {
+        ANIFEM_HIP_CHECK(hipMemcpyAsync(nnz, rp + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    }
+    ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
+    if (hw) *nnz = hw[0], *groups = hw[1];
+    return ANIFEM_OK;
+}
 
 constexpr size_t kSmallEntries = (size_t)kSmallChunks * 64 * kSmallChunk;
 size_t small_bytes() { return kSmallEntries * (sizeof(double) + sizeof(uint16_t)); }
@@ -1252,8 +1293,7 @@ int launch_small(int64_t n, const int64_t* rp, const int32_t* ci, const double* 
     return ANIFEM_OK;
 }
 
-// Final report: the true residual ||b - A x|| from x, and the state's counters
-// (kNotTaken: the one-workgroup solver left x as it was).
+// Final report: the true residual ||b - A x|| from x, and the state's counters.
 int finish(int64_t n, int64_t nnz, const int64_t* rp, const int32_t* ci, const double* v, const double* b,
            const double* x, double* Ax, double* part, const PcgState* st, anifem_pcg_result* res, hipStream_t s) {
     const unsigned vb = (unsigned)std::min<int64_t>((n + kThreads - 1) / kThreads, kRedBlocks);
@@ -1272,7 +1312,6 @@ int finish(int64_t n, int64_t nnz, const int64_t* rp, const int32_t* ci, const d
         res->relres = std::sqrt(hs.rr / hs.bb);
         res->true_relres = std::sqrt(tr / hs.bb);
     }
-    if (hs.done == kNotTaken) return kNotTaken;
     return hs.done ? ANIFEM_OK : ANIFEM_ERR_NOT_CONVERGED;
 }
 
@@ -1284,28 +1323,27 @@ extern "C" int anifem_pcg_jacobi(int64_t n, const int64_t* row_ptr, const int32_
     using namespace anifem;
     if (n <= 0 || !row_ptr || !col_idx || !val || !b || !x || rtol <= 0 || maxit < 0) return ANIFEM_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int64_t nnz = 0;
-    ANIFEM_HIP_CHECK(hipMemcpyAsync(&nnz, row_ptr + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    ANIFEM_HIP_CHECK(hipStreamSynchronize(s));
+    int64_t nnz = 0, groups = 0;
+    if (const int src = system_size(n, row_ptr, &nnz, &groups, s)) return src;
     double* work = nullptr;
     const size_t nv = (size_t)n;
     {
         const int wrc = workspace(0, sizeof(double) * (6 * nv + 3 * kRedBlocks) + sizeof(PcgState), (void**)&work);
         if (wrc) return wrc;
     }
-    if (small_system(n, nnz)) {
-        void* mat = nullptr;
-        int src = ANIFEM_OK;
-        if (workspace(2, small_bytes(), &mat)) {  // no room for the padded matrix: the launches below need none
-            (void)hipGetLastError();
-            src = kNotTaken;
-        }
+    void* mat = nullptr;
+    bool small = groups >= 0 && small_system(n, nnz, groups);
+    if (small && workspace(2, small_bytes(), &mat)) {  // no room for the padded matrix: the launches below need none
+        (void)hipGetLastError();
+        small = false;
+    }
+    if (small) {
         double *Ax = work, *part = work + nv;
         PcgState* st = reinterpret_cast<PcgState*>(part + kRedBlocks);
-        if (!src) src = launch_small(n, row_ptr, col_idx, val, b, x, rtol, maxit, mat, st, s);
+        int src = launch_small(n, row_ptr, col_idx, val, b, x, rtol, maxit, mat, st, s);
         if (!src) src = finish(n, nnz, row_ptr, col_idx, val, b, x, Ax, part, st, res, s);
         if (src != ANIFEM_OK) (void)hipStreamSynchronize(s);  // the workspace is idle on return
-        if (src != kNotTaken) return src;
+        return src;
     }
     double *r = work, *z = r + nv, *pb[2] = {z + nv, z + 2 * nv}, *Ap = z + 3 * nv, *dinv = Ap + nv, *part = dinv + nv;
     PcgState* st = reinterpret_cast<PcgState*>(part + 3 * kRedBlocks);
