@@ -907,9 +907,9 @@ __global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const i
     const double bb = s3[2] > 0 ? s3[2] : 1.0, tol2 = rtol * rtol * bb;
     // p_0 = z_0; iteration k as in dir_spmv / update_jacobi
     double beta = 0;
-    int64_t k = 0;
+    int64_t k = 0, last = rr == rr ? maxit : min(maxit, (int64_t)2);
     bool done = rr <= tol2;
-    while (!done && k < maxit) {
+    while (!done && k < last) {
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const int row = 64 * (w + kSmallWaves * i) + l;
@@ -942,6 +942,9 @@ __global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const i
         rr = s2[1];
         ++k;
         done = rr <= tol2;
+        // a NaN in r is in all of r, p and x after one more iteration, and the
+        // iterations up to maxit would change nothing more
+        if (rr != rr) last = min(last, k + 2);
     }
 #pragma unroll
     for (int i = 0; i < R; ++i) {
@@ -952,7 +955,7 @@ __global__ __launch_bounds__(kSmallThreads) void pcg_small_kernel(int n, const i
         st->rr = rr;
         st->bb = bb;
         st->tol2 = tol2;
-        st->it = k;
+        st->it = done ? k : maxit;
         st->done = done ? 1 : 0;
     }
 }
