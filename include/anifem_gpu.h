@@ -316,7 +316,7 @@ typedef struct anifem_block_layout {
     int64_t n_blocks;
     int64_t n_pairs;
     int64_t n_values;         /* element entries kept in the pattern, all blocks */
-    int64_t max_block_pairs;
+    int64_t max_block_pairs;  /* pairs, or rows where nodes outside every cell leave rows without one */
     int64_t max_block_values;
     int64_t max_block_slots;
 } anifem_block_layout;

@@ -49,23 +49,27 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
         }
     });
 
-    // greedy cut: extend the current block while every budget holds
+    // greedy cut: extend the current block while every budget holds.  A block has
+    // no more rows than the pairs' budget either: the passes hold one row start
+    // per lane, and a node that no cell uses has rows without a pair.
     S.blk_row0.assign(1, 0);
     S.blk_p0.assign(1, 0);
     S.blk_v0.assign(1, 0);
     {
-        int64_t slots = 0, nv = 0, np = 0;
+        int64_t slots = 0, nv = 0, np = 0, nr = 0;
         auto close = [&](int64_t r) {
             S.blk_row0.push_back((int32_t)r);
             S.blk_p0.push_back(S.blk_p0.back() + np);
             S.blk_v0.push_back(S.blk_v0.back() + nv);
-            slots = nv = np = 0;
+            slots = nv = np = nr = 0;
         };
         for (int64_t r = 0; r < ND; ++r) {
             const int64_t rs = S.row_ptr[r + 1] - S.row_ptr[r], rv = row_nv[r], rp = aptr[r + 1] - aptr[r];
             if (rs > caps.max_slots || rv > caps.max_values || rp > caps.max_pairs) return ANIFEM_ERR_DIMS;
-            if (slots && (slots + rs > caps.max_slots || nv + rv > caps.max_values || np + rp > caps.max_pairs))
+            if (slots && (slots + rs > caps.max_slots || nv + rv > caps.max_values || np + rp > caps.max_pairs ||
+                          nr + 1 > caps.max_pairs))
                 close(r);
+            ++nr;
             slots += rs;
             nv += rv;
             np += rp;
@@ -157,7 +161,8 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
     }
     for (int64_t b = 0; b < S.n_blocks; ++b) {
         S.max_block_values = std::max(S.max_block_values, S.blk_v0[b + 1] - S.blk_v0[b]);
-        S.max_block_pairs = std::max(S.max_block_pairs, S.blk_p0[b + 1] - S.blk_p0[b]);
+        S.max_block_pairs = std::max({S.max_block_pairs, S.blk_p0[b + 1] - S.blk_p0[b],
+                                      (int64_t)S.blk_row0[b + 1] - S.blk_row0[b]});
         S.max_block_slots = std::max(S.max_block_slots, S.blk_s0[b + 1] - S.blk_s0[b]);
     }
     return ANIFEM_OK;

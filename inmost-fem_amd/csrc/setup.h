@@ -18,7 +18,7 @@ namespace anifem {
 struct BlockCaps {
     int max_slots = 2048;   // CSR slots per block (<= 65535)
     int max_values = 2048;  // element entries per block (<= 65535)
-    int max_pairs = 256;    // (row, incident tet) pairs per block (<= workgroup size)
+    int max_pairs = 256;    // (row, incident tet) pairs, and rows, per block (<= workgroup size)
 };
 // Default budgets by entries per (row, tet) pair: a block of 256 pairs of nf
 // entries needs about 256 nf values, so larger element matrices get larger
@@ -129,7 +129,8 @@ struct AssemblySetup {
     std::vector<uint16_t> pair_pos;   // per pair, nf: value-list position of entry (ib, ia), or kPosDropped
     std::vector<uint16_t> sstart;     // nnz: first value of each slot, relative to its block
     std::vector<uint16_t> pstart;     // ndof: first pair of each row, relative to its block
-    int64_t max_block_values = 0, max_block_pairs = 0, max_block_slots = 0;
+    int64_t max_block_values = 0, max_block_slots = 0;
+    int64_t max_block_pairs = 0;  // pairs or, where rows have none, rows
 };
 
 int build_setup(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob, AssemblySetup& S,
