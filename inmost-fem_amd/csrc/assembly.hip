@@ -644,84 +644,68 @@ int greedy_colour(int64_t n_nodes, int64_t n_tets, const int32_t* tets, std::vec
 // The setup of a context: its enumeration phase on the device for a device
 // context, on the host for a host-only one (identical results).
 int build_host(anifem_assembly* ctx, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob,
-               const anifem::BlockCaps* caps = nullptr, bool on_device = false, void* stream = nullptr,
+               const anifem::BlockLadder& ladder, bool on_device = false, void* stream = nullptr,
                const anifem_vars_desc* vars = nullptr) {
     using namespace anifem;
     if (!mesh || !prob || !mesh->coords || !mesh->tets) return ANIFEM_ERR_ARG;
     if (vars) {
         // a multi-variable problem: element matrices only, numbering on the host
         if (vars->n_var < 1 || vars->n_var > kMaxVars) return ANIFEM_ERR_ARG;
-        int nf = 0;
-        for (int v = 0; v < vars->n_var; ++v) {
+        for (int v = 0; v < vars->n_var; ++v)
             if (!space_layout(vars->var[v].fem).valid || vars->var[v].ncomp < 1) return ANIFEM_ERR_ARG;
-            nf += nf_scalar(vars->var[v].fem) * vars->var[v].ncomp;
-        }
         ctx->prob = *prob;
         ctx->prob.dirichlet_dof_mask = nullptr;
         ctx->prob.trial = ctx->prob.test = anifem_op{ANIFEM_IDEN, vars->var[0].fem, vars->var[0].ncomp};
         ctx->vars_only = true;
-        const BlockCaps c = caps ? *caps : default_caps(nf, false);
-        const int rc = build_setup_vars(*mesh, vars->n_var, vars->var, *prob, ctx->S, c);
-        if (rc != ANIFEM_ERR_DIMS || caps) return rc;
-        ctx->S = AssemblySetup();  // the default budgets, then wider ones when one row exceeds them
-        return build_setup_vars(*mesh, vars->n_var, vars->var, *prob, ctx->S, wide_caps(nf));
+        return build_setup_vars(*mesh, vars->n_var, vars->var, *prob, ctx->S, ladder);
     }
     if (!op_valid(prob->trial) || !op_valid(prob->test)) return ANIFEM_ERR_ARG;
     // the global assembly numbers the DOFs of the spaces of space_layout
     if (!space_layout(prob->trial.fem).valid || !space_layout(prob->test.fem).valid) return ANIFEM_ERR_ARG;
     ctx->prob = *prob;
     ctx->prob.dirichlet_dof_mask = nullptr;
-    const int nf = nf_scalar(prob->test.fem) * prob->test.ncomp;
-    auto build = [&](const BlockCaps& c) {
-        return on_device ? build_setup_device(*mesh, *prob, ctx->S, c, stream) : build_setup(*mesh, *prob, ctx->S, c);
-    };
-    if (caps) return build(*caps);
-    int rc = ANIFEM_ERR_DIMS;
-    for (const BlockCaps& c : caps_ladder(nf, *prob, false)) {
-        ctx->S = AssemblySetup();
-        if ((rc = build(c)) != ANIFEM_ERR_DIMS) break;
-    }
-    return rc;
+    return on_device ? build_setup_device(*mesh, *prob, ctx->S, ladder, stream) : build_setup(*mesh, *prob, ctx->S, ladder);
 }
 
 }  // namespace
 
 namespace anifem {
 int assembly_create_caps(anifem_assembly** out, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob,
-                         const BlockCaps& caps, void* stream, const anifem_vars_desc* vars = nullptr);
+                         const BlockLadder& ladder, void* stream, const anifem_vars_desc* vars = nullptr);
 }
 
 namespace {
-// The default budgets, then wider ones when a single row exceeds them.
-int create_default(anifem_assembly** out, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob, int nf,
-                   void* stream, const anifem_vars_desc* vars) {
+// The default budgets of a problem of one space or several variables; empty for
+// one that is refused.
+anifem::BlockLadder default_ladder(const anifem_problem_desc* prob, const anifem_vars_desc* vars) {
     using namespace anifem;
-    if (!prob) return ANIFEM_ERR_ARG;
-    int rc = ANIFEM_ERR_DIMS;
-    for (const BlockCaps& c : caps_ladder(nf, *prob, vars != nullptr))
-        if ((rc = assembly_create_caps(out, mesh, prob, c, stream, vars)) != ANIFEM_ERR_DIMS) break;
-    return rc;
+    if (!prob) return {};
+    if (!vars) {
+        if (!op_valid(prob->test) || !space_layout(prob->test.fem).valid) return {};
+        return caps_ladder(nf_scalar(prob->test.fem) * prob->test.ncomp, *prob, false);
+    }
+    if (vars->n_var < 1 || vars->n_var > kMaxVars) return {};
+    int nf = 0;
+    for (int v = 0; v < vars->n_var; ++v) {
+        if (!space_layout(vars->var[v].fem).valid || vars->var[v].ncomp < 1) return {};
+        nf += nf_scalar(vars->var[v].fem) * vars->var[v].ncomp;
+    }
+    return caps_ladder(nf, *prob, true);
 }
 }  // namespace
 
 extern "C" int anifem_assembly_create_vars(anifem_assembly** out, const anifem_mesh_desc* mesh,
                                            const anifem_vars_desc* vars, const anifem_problem_desc* prob,
                                            void* stream) {
-    using namespace anifem;
-    if (!vars || vars->n_var < 1 || vars->n_var > kMaxVars) return ANIFEM_ERR_ARG;
-    int nf = 0;
-    for (int v = 0; v < vars->n_var; ++v) {
-        if (!space_layout(vars->var[v].fem).valid || vars->var[v].ncomp < 1) return ANIFEM_ERR_ARG;
-        nf += nf_scalar(vars->var[v].fem) * vars->var[v].ncomp;
-    }
-    return create_default(out, mesh, prob, nf, stream, vars);
+    if (!vars) return ANIFEM_ERR_ARG;
+    const anifem::BlockLadder ladder = default_ladder(prob, vars);
+    return ladder.empty() ? ANIFEM_ERR_ARG : anifem::assembly_create_caps(out, mesh, prob, ladder, stream, vars);
 }
 
 extern "C" int anifem_assembly_create(anifem_assembly** out, const anifem_mesh_desc* mesh,
                                       const anifem_problem_desc* prob, void* stream) {
-    if (!prob || !anifem::op_valid(prob->test) || !anifem::space_layout(prob->test.fem).valid) return ANIFEM_ERR_ARG;
-    const int nf = anifem::nf_scalar(prob->test.fem) * prob->test.ncomp;
-    return create_default(out, mesh, prob, nf, stream, nullptr);
+    const anifem::BlockLadder ladder = default_ladder(prob, nullptr);
+    return ladder.empty() ? ANIFEM_ERR_ARG : anifem::assembly_create_caps(out, mesh, prob, ladder, stream);
 }
 
 extern "C" int anifem_assembly_create_budget(anifem_assembly** out, const anifem_mesh_desc* mesh,
@@ -731,17 +715,17 @@ extern "C" int anifem_assembly_create_budget(anifem_assembly** out, const anifem
     c.max_slots = max_slots;
     c.max_values = max_values;
     c.max_pairs = max_pairs;
-    return anifem::assembly_create_caps(out, mesh, prob, c, stream);
+    return anifem::assembly_create_caps(out, mesh, prob, {c}, stream);
 }
 
 // Assembly context with given row-block budgets (the batch autotuner's trials).
 int anifem::assembly_create_caps(anifem_assembly** out, const anifem_mesh_desc* mesh,
-                                 const anifem_problem_desc* prob, const BlockCaps& caps, void* stream,
+                                 const anifem_problem_desc* prob, const BlockLadder& ladder, void* stream,
                                  const anifem_vars_desc* vars) {
     using namespace anifem;
     if (!out) return ANIFEM_ERR_ARG;
     std::unique_ptr<anifem_assembly> ctx(new anifem_assembly());
-    int rc = build_host(ctx.get(), mesh, prob, &caps, true, stream, vars);
+    int rc = build_host(ctx.get(), mesh, prob, ladder, true, stream, vars);
     if (rc) return rc;
     AssemblySetup& S = ctx->S;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -845,7 +829,9 @@ int anifem_assembly_create_host(anifem_assembly** out, const anifem_mesh_desc* m
     if (!out) return ANIFEM_ERR_ARG;
     std::unique_ptr<anifem_assembly> ctx(new anifem_assembly());
     ctx->host_only = true;
-    int rc = build_host(ctx.get(), mesh, prob);
+    const anifem::BlockLadder ladder = default_ladder(prob, nullptr);
+    if (ladder.empty()) return ANIFEM_ERR_ARG;
+    int rc = build_host(ctx.get(), mesh, prob, ladder);
     if (rc) return rc;
     *out = ctx.release();
     return ANIFEM_OK;
@@ -856,7 +842,9 @@ int anifem_assembly_create_vars_host(anifem_assembly** out, const anifem_mesh_de
     if (!out || !vars) return ANIFEM_ERR_ARG;
     std::unique_ptr<anifem_assembly> ctx(new anifem_assembly());
     ctx->host_only = true;
-    int rc = build_host(ctx.get(), mesh, prob, nullptr, false, nullptr, vars);
+    const anifem::BlockLadder ladder = default_ladder(prob, vars);
+    if (ladder.empty()) return ANIFEM_ERR_ARG;
+    int rc = build_host(ctx.get(), mesh, prob, ladder, false, nullptr, vars);
     if (rc) return rc;
     *out = ctx.release();
     return ANIFEM_OK;

@@ -40,7 +40,7 @@ namespace anifem {
 int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, anifem_status* status, hipStream_t s);
 int prepare_elem_args(const anifem_op& opA, const anifem_op& opB, const anifem_tensor* D, int order, ElemArgs& a);
 int assembly_create_caps(anifem_assembly** out, const anifem_mesh_desc* mesh, const anifem_problem_desc* prob,
-                         const BlockCaps& caps, void* stream, const anifem_vars_desc* vars = nullptr);
+                         const BlockLadder& ladder, void* stream, const anifem_vars_desc* vars = nullptr);
 }  // namespace anifem
 
 namespace {
@@ -145,7 +145,7 @@ int autotune_kind(anifem_batch* b, int kind, const anifem_batch_mesh& m, hipStre
     int rc = ANIFEM_OK;
     for (int c = 0; c < kCandidates && !rc; ++c) {
         anifem_assembly* ctx = nullptr;
-        rc = anifem::assembly_create_caps(&ctx, &md, &prob, kCandidateCaps[c], s);
+        rc = anifem::assembly_create_caps(&ctx, &md, &prob, {kCandidateCaps[c]}, s);
         if (rc == ANIFEM_ERR_DIMS) {  // a row does not fit this budget
             rc = ANIFEM_OK;
             b->tune_ms[kind][c] = -1;
@@ -525,7 +525,7 @@ int anifem_batch_create(anifem_batch** out, int n_meshes, const anifem_batch_mes
                     }
                     const anifem_batch_mesh& mj = meshes[j];
                     anifem_mesh_desc mdj{mj.n_nodes, mj.n_tets, mj.coords, mj.tets};
-                    rcs[j] = build_setup_device(mdj, problem_of(mj.fem, dirichlet), Ss[j], b->caps[kind_of(mj.fem)], ws);
+                    rcs[j] = build_setup_device(mdj, problem_of(mj.fem, dirichlet), Ss[j], {b->caps[kind_of(mj.fem)]}, ws);
                     if (!rcs[j]) p8_words[j] = compact_positions(Ss[j], P8[j]);
                     // what the concatenation does not read
                     std::vector<int32_t>().swap(Ss[j].slot);

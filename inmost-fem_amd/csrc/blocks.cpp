@@ -23,10 +23,11 @@
 namespace anifem {
 
 int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::vector<int32_t>& adj,
-                 const BlockCaps& caps) {
-    if (caps.max_slots < 1 || caps.max_slots > 65535 || caps.max_values < 1 || caps.max_values > 65535 ||
-        caps.max_pairs < 1 || caps.max_pairs > 256)
-        return ANIFEM_ERR_ARG;
+                 const BlockLadder& ladder) {
+    for (const BlockCaps& c : ladder)
+        if (c.max_slots < 1 || c.max_slots > 65535 || c.max_values < 1 || c.max_values > 65535 || c.max_pairs < 1 ||
+            c.max_pairs > 256)
+            return ANIFEM_ERR_ARG;
     const int64_t ND = S.ndof;
     const int nf = S.nf, E = S.E;
 
@@ -52,10 +53,10 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
     // greedy cut: extend the current block while every budget holds.  A block has
     // no more rows than the pairs' budget either: the passes hold one row start
     // per lane, and a node that no cell uses has rows without a pair.
-    S.blk_row0.assign(1, 0);
-    S.blk_p0.assign(1, 0);
-    S.blk_v0.assign(1, 0);
-    {
+    auto cut = [&](const BlockCaps& caps) {
+        S.blk_row0.assign(1, 0);
+        S.blk_p0.assign(1, 0);
+        S.blk_v0.assign(1, 0);
         int64_t slots = 0, nv = 0, np = 0, nr = 0;
         auto close = [&](int64_t r) {
             S.blk_row0.push_back((int32_t)r);
@@ -65,7 +66,7 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
         };
         for (int64_t r = 0; r < ND; ++r) {
             const int64_t rs = S.row_ptr[r + 1] - S.row_ptr[r], rv = row_nv[r], rp = aptr[r + 1] - aptr[r];
-            if (rs > caps.max_slots || rv > caps.max_values || rp > caps.max_pairs) return ANIFEM_ERR_DIMS;
+            if (rs > caps.max_slots || rv > caps.max_values || rp > caps.max_pairs) return false;
             if (slots && (slots + rs > caps.max_slots || nv + rv > caps.max_values || np + rp > caps.max_pairs ||
                           nr + 1 > caps.max_pairs))
                 close(r);
@@ -75,7 +76,9 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
             np += rp;
         }
         if (slots || ND == 0) close(ND);
-    }
+        return true;
+    };
+    if (!std::any_of(ladder.begin(), ladder.end(), cut)) return ANIFEM_ERR_DIMS;
     S.n_blocks = (int64_t)S.blk_row0.size() - 1;
     S.blk_s0.resize(S.n_blocks + 1);
     for (int64_t b = 0; b <= S.n_blocks; ++b) S.blk_s0[b] = S.row_ptr[S.blk_row0[b]];

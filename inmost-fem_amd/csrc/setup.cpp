@@ -439,25 +439,25 @@ void dof_adjacency(const AssemblySetup& S, std::vector<int64_t>& aptr, std::vect
 }
 
 int build_setup_vars(const anifem_mesh_desc& mesh, int n_var, const anifem_op* vars, const anifem_problem_desc& prob,
-                     AssemblySetup& S, const BlockCaps& caps) {
+                     AssemblySetup& S, const BlockLadder& ladder) {
     int rc = setup_prepare_vars(mesh, n_var, vars, S);
     if (!rc) rc = setup_enumerate_host(prob, S);
     if (rc) return rc;
     std::vector<int64_t> aptr;
     std::vector<int32_t> adj;
     dof_adjacency(S, aptr, adj);
-    return build_blocks(S, aptr, adj, caps);
+    return build_blocks(S, aptr, adj, ladder);
 }
 
 int build_setup(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob, AssemblySetup& S,
-                const BlockCaps& caps) {
+                const BlockLadder& ladder) {
     int rc = setup_prepare(mesh, prob, S);
     if (!rc) rc = setup_enumerate_host(prob, S);
     if (rc) return rc;
     std::vector<int64_t> aptr;
     std::vector<int32_t> adj;
     dof_adjacency(S, aptr, adj);
-    return build_blocks(S, aptr, adj, caps);
+    return build_blocks(S, aptr, adj, ladder);
 }
 
 }  // namespace anifem

@@ -63,7 +63,7 @@ inline BlockCaps wide_caps(int nf) {
     c.max_values = nf > 20 ? 16384 : 8192;
     return c;
 }
-// The budgets to try in turn, each where a single row exceeds the one before.
+// The default budgets of a problem, to be tried in turn.
 inline std::vector<BlockCaps> caps_ladder(int nf, const anifem_problem_desc& prob, bool vars) {
     const int ncomp = vars ? 0 : prob.test.ncomp;  // several variables: the budgets of a vector space
     std::vector<BlockCaps> c;
@@ -133,8 +133,11 @@ struct AssemblySetup {
     int64_t max_block_pairs = 0;  // pairs or, where rows have none, rows
 };
 
+// The block budgets of a setup, each tried where a single row exceeds the one
+// before (ANIFEM_ERR_DIMS after the last).
+using BlockLadder = std::vector<BlockCaps>;
 int build_setup(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob, AssemblySetup& S,
-                const BlockCaps& caps = BlockCaps());
+                const BlockLadder& ladder);
 // The phases of build_setup: argument checks and the node reorder; the
 // enumeration, Dirichlet flags, CSR pattern and slot map (host or device, with
 // identical results); the DOF -> tet adjacency the row blocks are cut from.
@@ -143,16 +146,16 @@ int setup_prepare(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob,
 // problem's trial and test are not used.
 int setup_prepare_vars(const anifem_mesh_desc& mesh, int n_var, const anifem_op* vars, AssemblySetup& S);
 int build_setup_vars(const anifem_mesh_desc& mesh, int n_var, const anifem_op* vars, const anifem_problem_desc& prob,
-                     AssemblySetup& S, const BlockCaps& caps = BlockCaps());
+                     AssemblySetup& S, const BlockLadder& ladder);
 int setup_enumerate_host(const anifem_problem_desc& prob, AssemblySetup& S);
 int setup_enumerate_device(const anifem_problem_desc& prob, AssemblySetup& S, void* stream);
 void dof_adjacency(const AssemblySetup& S, std::vector<int64_t>& aptr, std::vector<int32_t>& adj);
 // build_setup with the enumeration phase on the current device (stream-ordered
 // on `stream`); the host phase runs instead for meshes beyond its index ranges.
 int build_setup_device(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob, AssemblySetup& S,
-                       const BlockCaps& caps, void* stream);
+                       const BlockLadder& ladder, void* stream);
 int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::vector<int32_t>& adj,
-                 const BlockCaps& caps);
+                 const BlockLadder& ladder);
 // Compact value positions: per pair, the smallest kept position as 16 bits
 // and each entry's offset from it as one byte (0xFF: dropped), little endian
 // in ceil((2 + nf) / 4) 32-bit words.  Returns the words per pair, or 0 (out

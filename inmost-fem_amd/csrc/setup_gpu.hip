@@ -433,7 +433,7 @@ int setup_enumerate_device(const anifem_problem_desc& prob, AssemblySetup& S, vo
 namespace anifem {
 
 int build_setup_device(const anifem_mesh_desc& mesh, const anifem_problem_desc& prob, AssemblySetup& S,
-                       const BlockCaps& caps, void* stream) {
+                       const BlockLadder& ladder, void* stream) {
     int rc = setup_prepare(mesh, prob, S);
     if (rc) return rc;
     rc = setup_enumerate_device(prob, S, stream);
@@ -442,7 +442,7 @@ int build_setup_device(const anifem_mesh_desc& mesh, const anifem_problem_desc& 
     std::vector<int64_t> aptr;
     std::vector<int32_t> adj;
     dof_adjacency(S, aptr, adj);
-    return build_blocks(S, aptr, adj, caps);
+    return build_blocks(S, aptr, adj, ladder);
 }
 
 }  // namespace anifem
