@@ -37,6 +37,7 @@ struct anifem_assembly {
     int32_t* d_tetnodes = nullptr;    // 4 x n_tets SoA
     int32_t* d_blk_row0 = nullptr;
     anifem::BlockMeta* d_blk_meta = nullptr;
+    anifem::BlockMeta* d_blk_meta2 = nullptr;
     int64_t* d_blk_s0 = nullptr;
     int64_t* d_blk_p0 = nullptr;
     int64_t* d_blk_v0 = nullptr;
@@ -754,6 +755,7 @@ int anifem::assembly_create_caps(anifem_assembly** out, const anifem_mesh_desc* 
     if ((rc = upload(&ctx->d_tetnodes, tn.data(), tn.size(), s))) return rc;
     if ((rc = upload(&ctx->d_blk_row0, S.blk_row0.data(), S.blk_row0.size(), s))) return rc;
     if ((rc = upload(&ctx->d_blk_meta, S.blk_meta.data(), S.blk_meta.size(), s))) return rc;
+    if (!S.blk_meta2.empty() && (rc = upload(&ctx->d_blk_meta2, S.blk_meta2.data(), S.blk_meta2.size(), s))) return rc;
     if ((rc = upload(&ctx->d_blk_s0, S.blk_s0.data(), S.blk_s0.size(), s))) return rc;
     if ((rc = upload(&ctx->d_blk_p0, S.blk_p0.data(), S.blk_p0.size(), s))) return rc;
     if ((rc = upload(&ctx->d_blk_v0, S.blk_v0.data(), S.blk_v0.size(), s))) return rc;
@@ -860,7 +862,7 @@ int anifem_assembly_destroy(anifem_assembly* ctx) {
                         ctx->d_pstart,   ctx->d_row_ptr,  ctx->d_col_idx,  ctx->d_status,   ctx->d_kbuf,
                         ctx->d_slot,     ctx->d_dofs,     ctx->d_isdir,    ctx->d_plain_tab, ctx->d_col_tets,
                         ctx->d_lift,     ctx->d_pair_pos8, ctx->d_sign,   ctx->d_xyz,      ctx->d_ebuf,
-                        ctx->d_fbuf,     ctx->d_signmask, ctx->d_deg};
+                        ctx->d_fbuf,     ctx->d_signmask, ctx->d_deg,     ctx->d_blk_meta2};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
     }
@@ -1058,6 +1060,18 @@ void set_block_lists(const anifem_assembly* ctx, anifem::BlockArgs& a) {
     a.max_values = (int)S.max_block_values;
     a.max_pairs = (int)S.max_block_pairs;
     a.max_slots = (int)S.max_block_slots;
+}
+
+// The context's blocks in twos, where it has them.
+bool take_in_twos(const anifem_assembly* ctx, anifem::BlockArgs& a) {
+    if (!ctx->d_blk_meta2) return false;
+    const anifem::AssemblySetup& S = ctx->S;
+    a.meta = ctx->d_blk_meta2;
+    a.n_blocks = (int64_t)S.blk_meta2.size();
+    a.max_values = S.meta2_max.max_values;
+    a.max_pairs = S.meta2_max.max_pairs;
+    a.max_slots = S.meta2_max.max_slots;
+    return true;
 }
 
 // RT0 / ND0 with one operator on both sides and tensors constant over each
@@ -1305,13 +1319,15 @@ int anifem_assembly_run_rhs(anifem_assembly* ctx, const void* F_elem, int elem_p
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, ctx->d_status, 4);
     ANIFEM_HIP_CHECK(hipGetLastError());
     if (S.n_blocks > 0) {
-        const unsigned grid = (unsigned)(8 * ((S.n_blocks + 7) / 8));
-        if (elem_precision == ANIFEM_PREC_FP64)
-            hipLaunchKernelGGL(row_block_rhs_kernel<double>, dim3(grid), dim3(kBlock), 0, s, a,
-                               static_cast<const double*>(F_elem), accumulate ? 1 : 0);
-        else
-            hipLaunchKernelGGL(row_block_rhs_kernel<float>, dim3(grid), dim3(kBlock), 0, s, a,
-                               static_cast<const float*>(F_elem), accumulate ? 1 : 0);
+        const bool two = take_in_twos(ctx, a);
+        const unsigned grid = (unsigned)(8 * ((a.n_blocks + 7) / 8));
+        auto launch = [&](auto* F) {
+            typedef std::decay_t<decltype(*F)> TE;
+            hipLaunchKernelGGL((two ? row_block_rhs_kernel<TE, true> : row_block_rhs_kernel<TE, false>), dim3(grid),
+                               dim3(kBlock), 0, s, a, F, accumulate ? 1 : 0);
+        };
+        if (elem_precision == ANIFEM_PREC_FP64) launch(static_cast<const double*>(F_elem));
+        else launch(static_cast<const float*>(F_elem));
         ANIFEM_HIP_CHECK(hipGetLastError());
     }
     return status ? read_status(nullptr, 0, ctx->d_status, true, status, s) : ANIFEM_OK;
@@ -1351,20 +1367,31 @@ namespace {
 
 // Persistent element scatter for the common element sizes (occupancy x CUs
 // workgroups, whole XCD groups), else one workgroup per block.
-template <typename TE, int NF, bool SYM>
-int launch_elements_persistent(anifem_assembly* ctx, const anifem::BlockArgs& a, const TE* A, const TE* F, size_t lds,
-                               hipStream_t s) {
+template <typename TE, int NF, bool SYM, bool TWO>
+int launch_elements_blocks(anifem_assembly* ctx, const anifem::BlockArgs& a, const TE* A, const TE* F, hipStream_t s) {
     using namespace anifem;
+    const size_t lds = block_lds_layout(a.max_values, a.max_pairs, a.max_slots, 8, 0, 0).total;
     int occ = 0, n_cu = 0;
     ANIFEM_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &occ, reinterpret_cast<const void*>(&row_block_elements_persistent<TE, NF, SYM>), kBlock, lds));
+        &occ, reinterpret_cast<const void*>(&row_block_elements_persistent<TE, NF, SYM, TWO>), kBlock, lds));
     ANIFEM_HIP_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device));
     int64_t G = (int64_t)std::max(occ, 1) * std::max(n_cu, 1);
-    G = std::min<int64_t>(G, ctx->S.n_blocks);
+    G = std::min<int64_t>(G, a.n_blocks);
     G = std::max<int64_t>(8, G / 8 * 8);
-    hipLaunchKernelGGL((row_block_elements_persistent<TE, NF, SYM>), dim3((unsigned)G), dim3(kBlock), lds, s, a, A, F);
+    hipLaunchKernelGGL((row_block_elements_persistent<TE, NF, SYM, TWO>), dim3((unsigned)G), dim3(kBlock), lds, s, a, A,
+                       F);
     ANIFEM_HIP_CHECK(hipGetLastError());
     return ANIFEM_OK;
+}
+
+// General P2^3 matrices take the context's blocks in twos, where it has them
+// (BlockMeta::set_first).
+template <typename TE, int NF, bool SYM>
+int launch_elements_persistent(anifem_assembly* ctx, anifem::BlockArgs a, const TE* A, const TE* F, hipStream_t s) {
+    if constexpr (NF == 30 && !SYM) {
+        if (take_in_twos(ctx, a)) return launch_elements_blocks<TE, NF, SYM, true>(ctx, a, A, F, s);
+    }
+    return launch_elements_blocks<TE, NF, SYM, false>(ctx, a, A, F, s);
 }
 
 template <typename TE, bool SYM>
@@ -1373,11 +1400,11 @@ int launch_elements(anifem_assembly* ctx, const anifem::BlockArgs& a, const TE* 
     using namespace anifem;
     if (ctx->persistent) {
         switch (ctx->S.nf) {
-            case 4: return launch_elements_persistent<TE, 4, SYM>(ctx, a, A, F, lds, s);
-            case 10: return launch_elements_persistent<TE, 10, SYM>(ctx, a, A, F, lds, s);
-            case 12: return launch_elements_persistent<TE, 12, SYM>(ctx, a, A, F, lds, s);
-            case 20: return launch_elements_persistent<TE, 20, SYM>(ctx, a, A, F, lds, s);
-            case 30: return launch_elements_persistent<TE, 30, SYM>(ctx, a, A, F, lds, s);
+            case 4: return launch_elements_persistent<TE, 4, SYM>(ctx, a, A, F, s);
+            case 10: return launch_elements_persistent<TE, 10, SYM>(ctx, a, A, F, s);
+            case 12: return launch_elements_persistent<TE, 12, SYM>(ctx, a, A, F, s);
+            case 20: return launch_elements_persistent<TE, 20, SYM>(ctx, a, A, F, s);
+            case 30: return launch_elements_persistent<TE, 30, SYM>(ctx, a, A, F, s);
             default: break;
         }
     }

@@ -734,14 +734,17 @@ __global__ __launch_bounds__(kBlock) void row_block_elements_kernel(BlockArgs a,
 // block; each pair's load-vector entry (0 on a Dirichlet row, applyDir) goes
 // to LDS, then one lane per row adds its pairs' entries in ascending tet order
 // and stores (accumulate = 0) or adds the sum to rhs (rhs <- rhs + assembled).
-template <typename TE>
+// TWO: records of two blocks (blk_meta2).  A workgroup is a chain of dependent
+// loads: with 128 pairs in each, P2^3 at 44^3 took 111 us (FP64) against 72.
+template <typename TE, bool TWO>
 __global__ __launch_bounds__(kBlock) void row_block_rhs_kernel(BlockArgs a, const TE* __restrict__ Fe, int accumulate) {
     __shared__ double fv[kBlock];
     const int64_t per_xcd = (a.n_blocks + 7) / 8;
     const int64_t k = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (k >= a.n_blocks) return;  // uniform over the workgroup
     const BlockMeta M = a.meta[k];
-    const int nf = a.kinds[M.kind].nf;
+    const int nf = a.kinds[0].nf;
+    const int nr1 = TWO ? M.nr1() : M.nr, np1 = TWO ? M.np1() : 0;
     int nonfinite = 0;
     if ((int)threadIdx.x < M.np) {
         const int64_t gp = M.p0 + threadIdx.x;
@@ -755,8 +758,8 @@ __global__ __launch_bounds__(kBlock) void row_block_rhs_kernel(BlockArgs a, cons
     }
     __syncthreads();
     for (int u = threadIdx.x; u < M.nr; u += kBlock) {
-        const int pb = a.pstart[M.r0 + u];
-        const int pe = u + 1 < M.nr ? a.pstart[M.r0 + u + 1] : M.np;
+        const int pb = a.pstart[M.r0 + u] + (u >= nr1 ? np1 : 0);
+        const int pe = u + 1 < M.nr ? a.pstart[M.r0 + u + 1] + (u + 1 >= nr1 ? np1 : 0) : M.np;
         double sum = 0.0;
         for (int p = pb; p < pe; ++p) sum += fv[p];
         a.rhs[M.r0 + u] = accumulate ? a.rhs[M.r0 + u] + sum : sum;
@@ -1388,7 +1391,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(SPLIT ? 
 // records in flight during phase A and its matrix rows, load-vector entries,
 // slot and row starts requested after it.  Phase A only places values, so
 // the results are bitwise those of row_block_elements_kernel.
-template <typename TE, int NF, bool SYM>
+// TWO: records of two blocks (blk_meta2).  A general matrix's row is one entry of
+// every column, and the rows of one tet share those lines within a block: P2^3 at
+// 44^3 in FP64 4.24 ms with 128 pairs to a workgroup against 4.04 (128 lanes each: 4.7).
+template <typename TE, int NF, bool SYM, bool TWO>
 __global__ __launch_bounds__(kBlock) void row_block_elements_persistent(BlockArgs a, const TE* __restrict__ Ae,
                                                                         const TE* __restrict__ Fe) {
     constexpr int PW = NF / 2;
@@ -1481,7 +1487,9 @@ __global__ __launch_bounds__(kBlock) void row_block_elements_persistent(BlockArg
         if (bnn >= 0) Mnn = a.meta[bnn];
 
         // phase A of b: the pair's row placed at its listed positions
+        const int nv1 = TWO ? M.nv1() : 0, ns1 = TWO ? M.ns1() : 0, nr1 = TWO ? M.nr1() : 0, np1 = TWO ? M.np1() : 0;
         if ((int)threadIdx.x < M.np) {
+            double* pv = TWO && (int)threadIdx.x >= np1 ? vals + nv1 : vals;
             const bool dir = (cur.ibf & kPairDirichlet) != 0;
 #pragma unroll
             for (int e = 0; e < NF; ++e) {
@@ -1490,7 +1498,7 @@ __global__ __launch_bounds__(kBlock) void row_block_elements_persistent(BlockArg
                 if (ps != kPosDropped) {
                     const double v = dir ? 1.0 : ((cur.flip >> e) & 1 ? -(double)cur.v[e] : (double)cur.v[e]);
                     nonfinite += isfinite(v) ? 0 : 1;
-                    vals[ps] = v;
+                    pv[ps] = v;
                 }
             }
             if (a.has_rhs) {
@@ -1505,8 +1513,8 @@ __global__ __launch_bounds__(kBlock) void row_block_elements_persistent(BlockArg
         // phase B of b
         const int ns = M.ns, nv = M.nv, nr = M.nr, np = M.np;
         for (int u = threadIdx.x; u < ns; u += kBlock) {
-            const int cb = sstb[u];
-            const int ce = u + 1 < ns ? sstb[u + 1] : nv;
+            const int cb = sstb[u] + (TWO && u >= ns1 ? nv1 : 0);
+            const int ce = u + 1 < ns ? sstb[u + 1] + (TWO && u + 1 >= ns1 ? nv1 : 0) : nv;
             double sum = 0.0;
             int c = cb;
             for (; c + 4 <= ce; c += 4) {
@@ -1521,8 +1529,8 @@ __global__ __launch_bounds__(kBlock) void row_block_elements_persistent(BlockArg
         }
         if (a.has_rhs) {
             for (int u = threadIdx.x; u < nr; u += kBlock) {
-                const int pb = pstl[u];
-                const int pe = u + 1 < nr ? pstl[u + 1] : np;
+                const int pb = pstl[u] + (TWO && u >= nr1 ? np1 : 0);
+                const int pe = u + 1 < nr ? pstl[u + 1] + (TWO && u + 1 >= nr1 ? np1 : 0) : np;
                 double sum = 0.0;
                 for (int p = pb; p < pe; ++p) sum += fvals[p];
                 a.rhs[M.r0 + u] = sum;

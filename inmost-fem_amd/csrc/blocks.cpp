@@ -17,6 +17,7 @@
 // vector entries are 0; such a pair carries kPairDirichlet.
 #include <algorithm>
 #include <atomic>
+#include <utility>
 
 #include "setup.h"
 
@@ -82,6 +83,12 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
     S.n_blocks = (int64_t)S.blk_row0.size() - 1;
     S.blk_s0.resize(S.n_blocks + 1);
     for (int64_t b = 0; b <= S.n_blocks; ++b) S.blk_s0[b] = S.row_ptr[S.blk_row0[b]];
+    for (int64_t b = 0; b < S.n_blocks; ++b) {
+        S.max_block_values = std::max(S.max_block_values, S.blk_v0[b + 1] - S.blk_v0[b]);
+        S.max_block_pairs = std::max({S.max_block_pairs, S.blk_p0[b + 1] - S.blk_p0[b],
+                                      (int64_t)S.blk_row0[b + 1] - S.blk_row0[b]});
+        S.max_block_slots = std::max(S.max_block_slots, S.blk_s0[b + 1] - S.blk_s0[b]);
+    }
 
     // fill the pair lists and value positions, one block at a time
     const int64_t NP = S.blk_p0.back();
@@ -90,7 +97,7 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
     S.pair_pos.resize((size_t)NP * nf);
     S.sstart.resize(S.nnz);
     S.pstart.resize(ND);
-    host_parallel_for(S.n_blocks, 16, [&](int64_t b0, int64_t b1) {
+    host_parallel_for(S.n_blocks, 32, [&](int64_t b0, int64_t b1) {
         std::vector<int32_t> cur;
         for (int64_t b = b0; b < b1; ++b) {
             const int32_t r0 = S.blk_row0[b], r1 = S.blk_row0[b + 1];
@@ -146,27 +153,44 @@ int build_blocks(AssemblySetup& S, const std::vector<int64_t>& aptr, const std::
         for (int64_t b = 0; b < S.n_blocks; ++b) S.blk_order[b] = (int32_t)b;
         std::stable_sort(S.blk_order.begin(), S.blk_order.end(),
                          [&](int32_t x, int32_t y) { return key[x] < key[y]; });
-        S.blk_meta.resize(S.n_blocks);
-        for (int64_t k = 0; k < S.n_blocks; ++k) {
-            const int64_t b = S.blk_order[k];
-            BlockMeta& M = S.blk_meta[k];
+        // the record of blocks b .. b + count - 1
+        auto record = [&](int64_t b, int64_t count) {
+            const int64_t e = b + count;
+            BlockMeta M{};
             M.s0 = S.blk_s0[b];
             M.p0 = S.blk_p0[b];
             M.q0 = S.blk_p0[b] * nf;
             M.r0 = S.blk_row0[b];
-            M.nr = (uint16_t)(S.blk_row0[b + 1] - S.blk_row0[b]);
-            M.ns = (uint16_t)(S.blk_s0[b + 1] - S.blk_s0[b]);
-            M.np = (uint16_t)(S.blk_p0[b + 1] - S.blk_p0[b]);
-            M.nv = (uint16_t)(S.blk_v0[b + 1] - S.blk_v0[b]);
-            M.kind = 0;
-            M.pad = 0;
+            M.nr = (uint16_t)(S.blk_row0[e] - S.blk_row0[b]);
+            M.ns = (uint16_t)(S.blk_s0[e] - S.blk_s0[b]);
+            M.np = (uint16_t)(S.blk_p0[e] - S.blk_p0[b]);
+            M.nv = (uint16_t)(S.blk_v0[e] - S.blk_v0[b]);
+            return M;
+        };
+        S.blk_meta.resize(S.n_blocks);
+        for (int64_t k = 0; k < S.n_blocks; ++k) S.blk_meta[k] = record(S.blk_order[k], 1);
+        if (nf == 30 && S.max_block_pairs <= 128) {
+            const BlockCaps two = default_caps(nf, false);
+            std::vector<std::pair<int64_t, BlockMeta>> m;
+            for (int64_t b = 0; b < S.n_blocks;) {
+                const bool fits = b + 1 < S.n_blocks && S.blk_s0[b + 2] - S.blk_s0[b] <= two.max_slots &&
+                                  S.blk_v0[b + 2] - S.blk_v0[b] <= two.max_values &&
+                                  S.blk_p0[b + 2] - S.blk_p0[b] <= two.max_pairs &&
+                                  S.blk_row0[b + 2] - S.blk_row0[b] <= two.max_pairs;
+                BlockMeta M = record(b, fits ? 2 : 1);
+                M.set_first(record(b, 1));
+                m.emplace_back(fits ? std::max(key[b], key[b + 1]) : key[b], M);
+                b += fits ? 2 : 1;
+            }
+            std::stable_sort(m.begin(), m.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+            S.meta2_max = BlockCaps{0, 0, 0};
+            for (const auto& [k, M] : m) {
+                S.blk_meta2.push_back(M);
+                S.meta2_max.max_slots = std::max<int>(S.meta2_max.max_slots, M.ns);
+                S.meta2_max.max_values = std::max<int>(S.meta2_max.max_values, M.nv);
+                S.meta2_max.max_pairs = std::max<int>({S.meta2_max.max_pairs, M.np, M.nr});
+            }
         }
-    }
-    for (int64_t b = 0; b < S.n_blocks; ++b) {
-        S.max_block_values = std::max(S.max_block_values, S.blk_v0[b + 1] - S.blk_v0[b]);
-        S.max_block_pairs = std::max({S.max_block_pairs, S.blk_p0[b + 1] - S.blk_p0[b],
-                                      (int64_t)S.blk_row0[b + 1] - S.blk_row0[b]});
-        S.max_block_slots = std::max(S.max_block_slots, S.blk_s0[b + 1] - S.blk_s0[b]);
     }
     return ANIFEM_OK;
 }

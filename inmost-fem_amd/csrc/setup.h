@@ -42,12 +42,12 @@ inline BlockCaps default_caps(int nf, bool scalar_space) {
 // Elasticity on three components of P2 (30 entries per pair, the compact Lame
 // rows) takes blocks of 128 pairs as well: two lanes per pair in the fused pass and
 // three workgroups per CU instead of two (48^3 cube: FP64 1.69 -> 1.56 ms, FP32
-// 1.57 -> 1.24).  The scatter of element matrices on these blocks went from 3.37 to
-// 2.59 ms (FP64 symmetric), 2.94 to 1.89 (FP32 symmetric), 4.41 to 4.08 (FP32
-// general) and 5.51 to 5.67 (FP64 general: whole-row gathers); other tensors, whose
-// pass holds the blocks of K in registers and stays at two workgroups, keep the
-// budgets of default_caps.  The slots stay within what the pass carries in
-// registers.
+// 1.57 -> 1.24).  The scatter of symmetric element matrices gains as well (44^3:
+// FP64 2.61 -> 1.99 ms, FP32 2.26 -> 1.45); that of general ones and the load
+// vectors, which lose by smaller blocks, take these in twos
+// (AssemblySetup::blk_meta2).  Other tensors, whose pass holds the blocks of K in
+// registers and stays at two workgroups, keep the budgets of default_caps.  The
+// slots stay within what the pass carries in registers.
 inline BlockCaps p2vec_caps() {
     BlockCaps c;
     c.max_slots = 2544;
@@ -87,6 +87,18 @@ struct BlockMeta {
     uint16_t np, nv;  // pairs, values
     uint32_t kind;    // index of the block's element kind (batched assembly), else 0
     uint32_t pad;
+    // A record of two blocks, consecutive in row order, that one workgroup takes
+    // as one (AssemblySetup::blk_meta2): the counts above are their sums, and
+    // these the first one's.  Positions, slot starts and pair starts of the second
+    // are relative to itself: np1, nv1 are to be added past ns1, nr1, np1.
+    __host__ __device__ void set_first(const BlockMeta& a) {
+        kind = a.np | (uint32_t)a.nv << 16;
+        pad = a.ns | (uint32_t)a.nr << 16;
+    }
+    __host__ __device__ int np1() const { return kind & 0xFFFF; }
+    __host__ __device__ int nv1() const { return kind >> 16; }
+    __host__ __device__ int ns1() const { return pad & 0xFFFF; }
+    __host__ __device__ int nr1() const { return pad >> 16; }
 };
 static_assert(sizeof(BlockMeta) == 48, "block metadata is one 48-byte record");
 
@@ -121,6 +133,11 @@ struct AssemblySetup {
     std::vector<int32_t> blk_row0;    // n_blocks + 1
     std::vector<int32_t> blk_order;   // n_blocks: processing order of the blocks
     std::vector<BlockMeta> blk_meta;  // n_blocks: bounds in processing order
+    // P2^3 blocks of at most 128 pairs (p2vec_caps) in twos, or alone where two
+    // exceed default_caps, for the passes that larger blocks suit better (load
+    // vectors, matrices read by whole rows): in processing order, else empty
+    std::vector<BlockMeta> blk_meta2;
+    BlockCaps meta2_max;              // the largest of them
     std::vector<int64_t> blk_s0;      // n_blocks + 1: first CSR slot of each block (row_ptr[blk_row0])
     std::vector<int64_t> blk_p0;      // n_blocks + 1 offsets into the pair lists
     std::vector<int64_t> blk_v0;      // n_blocks + 1 offsets of each block's value list
