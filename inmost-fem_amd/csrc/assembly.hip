@@ -159,8 +159,7 @@ static __global__ __launch_bounds__(kBlock) void publish_counts_kernel(const int
 // The status of the pass queued last on s, counts in d_status (and deg): written
 // by a launch to the thread's pinned words (a copy of 16 bytes from device
 // memory took longer than the small passes it reports on: the 16^3 P1 assembly
-// 38.5 us with it, 30.5 without; the batch of 32 uneven meshes 277 -> 274), or
-// copied where there are none.
+// 38.5 us with it, 30.5 without), or copied where there are none.
 int read_status(const int* deg, int64_t n_deg, int* d_status, bool may_alloc, anifem_status* status, hipStream_t s) {
     int* dw = nullptr;
     volatile int* hw = host_words(&dw, may_alloc);

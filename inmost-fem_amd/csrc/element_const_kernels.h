@@ -12,7 +12,7 @@
 //   * the lanes of consecutive tets store one contiguous range.
 // FP64 P2 with a symmetric tensor, 1,572,864 tets: 463 us -> 364 us (4.1 TB/s; with
 // 128 and 64 tets per workgroup 374 and 446 us); FP32 P2^3 elasticity, 663,552
-// tets: 952 us -> 512 us (4.8 TB/s; 969 us with nontemporal stores, which leave the
+// tets: 952 us -> 528 us (4.7 TB/s; 969 us with nontemporal stores, which leave the
 // columns' shared lines unmerged).
 #pragma once
 

@@ -711,13 +711,14 @@ __global__ __launch_bounds__(kThreads) void residual_kernel(int64_t n, const dou
 // ---- the whole solve in one workgroup (small systems) ----------------------
 // An iteration of a small system is a chain of latencies: two launches, each
 // reading row pointers, columns, operands and partial sums that the last launch
-// left beyond this chiplet's L2 (10.8 us at 4,913 rows).  One workgroup of 16
+// left beyond this chiplet's L2 (11.5 to 13 us at 4,913 rows).  One workgroup of 16
 // waves needs no launch: p stays in LDS, x, r, 1/diag and A p in registers (lane
 // = row, R rows per lane), and the matrix is streamed from L2 in the layout its
 // first pass writes: slices of 64 rows, as wide as their longest row in groups
 // of 8 entries; a group is four 16-byte loads of values and one of 16-bit columns
 // per lane, and the next group is in flight while one is used.  The rate at which
-// one CU reads L2 then bounds it (16^3 P1, 46,941 entries: 8.7 us an iteration with the call, from 13.2).
+// one CU reads L2 then bounds it (16^3 P1, 46,941 entries: 8.5 us an iteration, the
+// call included, where the launches take 11.5 to 13).
 // Sums run in a fixed order.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / 64;
@@ -1255,10 +1256,12 @@ int workspace(int slot, size_t bytes, void** out) {
 }
 
 // Systems the one-workgroup solver takes: rows within its LDS and registers
-// and a matrix that streams faster than two launches run: 46,941 entries of 16^3
-// P1 8.7 against 13.2 us an iteration, 51,109 of P2 at 7^3 (rows of 10 to 65, wider
-// slices) 14.9 against 14.7; at 4,437 entries 3.9 against 15.7.  Both sizes come
-// from row_ptr before anything else is queued.
+// and a matrix that streams faster than two launches run.  The load groups decide
+// that: 21 groups (P1 at 8^3) 3.8 against 14.9 us an iteration, 145 (16^3) 8.7
+// against 13.1, 144 (P2 at 6^3) 8.6 against 15.1; the limits lie on the safe side of
+// the break-even (with wider ones, 210 groups of P2 at 7^3 11.2 against 14.8, 312
+// at 8^3 14.8 against 15.2).  Both sizes come from row_ptr before anything else is
+// queued.
 bool small_system(int64_t n, int64_t nnz, int64_t groups) {
     return n <= kSmallRows && nnz <= kSmallNnz && groups <= kSmallChunks;
 }
