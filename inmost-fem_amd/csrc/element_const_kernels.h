@@ -105,18 +105,24 @@ __global__ __launch_bounds__(kBlock) void element_const_kernel(ElemArgs a) {
     }
     __syncthreads();
 
-    // L lanes per tet: VEC rows x the columns c, c + C, .. of every component
-    const int nfB = a.nfB0 * NCB, rows = nfB / VEC, C = (a.nfA0 + J - 1) / J, L = rows * C;
-    const int NG = L < kBlock ? kBlock / L : 1;
-    const int g = threadIdx.x / L;
-    if (g >= NG) return;
+    // a lane takes VEC rows x J columns of every component.  A matrix of more
+    // than kBlock such items (P3^3: 30 x 10) goes in passes of whole columns:
+    // J C of them from c0, over all tets, the tets dealt out to NG groups of lanes.
+    // Passes of kBlock items, broken inside columns, left a last one of 44 lanes and
+    // lines stored in two parts: P3^3 elasticity, 100,003 tets, FP64 692 -> 563 us
+    // (5.1 TB/s), FP32 458 -> 378 us
+    const int nfB = a.nfB0 * NCB, rows = nfB / VEC;
     const T* R = reinterpret_cast<const T*>(
         sizeof(T) == 8 ? static_cast<const void*>(SYM ? a.Rds : a.Rd) : static_cast<const void*>(SYM ? a.Rfs : a.Rf));
     struct alignas(VEC * sizeof(T)) Vec {
         T v[VEC];
     };
-    for (int item = threadIdx.x - g * L; item < L; item += kBlock) {
-        const int c = item / rows, ib = VEC * (item - c * rows), cb = ib / a.nfB0, ib0 = ib - cb * a.nfB0;
+    for (int c0 = 0, C; c0 < a.nfA0; c0 += J * C) {
+        C = (a.nfA0 - c0 + J - 1) / J;
+        if (C > kBlock / rows) C = kBlock / rows;
+        const int L = rows * C, NG = kBlock / L, g = threadIdx.x / L, item = threadIdx.x - g * L;
+        if (g >= NG) continue;
+        const int c = c0 + item / rows, ib = VEC * (item % rows), cb = ib / a.nfB0, ib0 = ib - cb * a.nfB0;
         T Rr[J][VEC][KBC];
 #pragma unroll
         for (int j = 0; j < J; ++j)

@@ -62,3 +62,13 @@ def test_const_kernel_shapes_match_oracle(pair, tt, n):
             assert (buf[shift + n * E:] == -7.0).all() and (buf[:shift] == -7.0).all()
             assert T.rel_frob(A[:m], ref) <= tol
             assert np.array_equal(A, A[cell])  # a cell's matrix does not depend on its place
+
+
+@pytest.mark.parametrize("pair,tt,n", [
+    ((2, 4, 3, 2, 4, 3), af.TENSOR_GENERAL, 1), ((1, 4, 3, 1, 4, 3), af.TENSOR_SCALAR, 37),
+    ((2, 4, 3, 2, 4, 3), af.TENSOR_SYMMETRIC, 512 * 32 + 1), ((1, 4, 1, 2, 4, 3), af.TENSOR_GENERAL, 51),
+    ((2, 4, 3, 1, 4, 1), af.TENSOR_GENERAL, 49), ((2, 3, 1, 2, 4, 3), af.TENSOR_GENERAL, 18)])
+def test_matrices_of_several_passes_match_oracle(pair, tt, n):
+    """More items than lanes: whole columns per pass, the last pass's cells dealt
+    out to groups of lanes."""
+    test_const_kernel_shapes_match_oracle(pair, tt, n)
