@@ -18,8 +18,15 @@ int launch(ElemArgs a, hipStream_t s) {
     // Cells per workgroup: 256 while five workgroups share a CU's LDS (the
     // stores of some then cover the geometry of the others); fewer for small
     // batches, whose time is the length of one workgroup's chain.
+    // The Piola spaces' geometry is long and its registers let three workgroups
+    // share a CU (so 48 KB each): between 384 and 768 of them, which one round
+    // holds, where 512 to 1,024 ran a second, and 256 cells also where 32 KB
+    // allowed 128 or 64.  RT0 IDEN, general tensor: 16,000 cells 17.1 -> 10.2 us,
+    // 100,003 25.8 -> 18.6; ND0 GRAD 600,000 168 -> 122.
+    const size_t lds_max = (PIOLA ? 48 : 32) * 1024;
+    const int64_t least = PIOLA ? 384 : 512;
     int tile = kBlock;
-    while (tile > 16 && (lds(tile) > 32 * 1024 || a.n < (int64_t)512 * tile)) tile /= 2;
+    while (tile > 16 && (lds(tile) > lds_max || a.n < least * tile)) tile /= 2;
     a.tile = tile;
     const dim3 grid((unsigned)((a.n + tile - 1) / tile));
     // row pairs need an even number of rows per component and an output

@@ -72,3 +72,10 @@ def test_matrices_of_several_passes_match_oracle(pair, tt, n):
     """More items than lanes: whole columns per pass, the last pass's cells dealt
     out to groups of lanes."""
     test_const_kernel_shapes_match_oracle(pair, tt, n)
+
+
+@pytest.mark.parametrize("pair,tt", [((1, 21, 1, 1, 21, 1), af.TENSOR_GENERAL), ((2, 25, 1, 2, 25, 1), af.TENSOR_SYMMETRIC),
+                                     ((4, 25, 1, 4, 25, 1), af.TENSOR_GENERAL)])
+@pytest.mark.parametrize("n", [384 * 32 - 1, 384 * 32, 384 * 128 + 5, 384 * 256 - 1, 384 * 256 + 1])
+def test_face_and_edge_spaces_either_side_of_a_change_of_cells_per_workgroup(pair, tt, n):
+    test_const_kernel_shapes_match_oracle(pair, tt, n)
