@@ -110,7 +110,8 @@ __global__ __launch_bounds__(kBlock) void element_const_kernel(ElemArgs a) {
     // J C of them from c0, over all tets, the tets dealt out to NG groups of lanes.
     // Passes of kBlock items, broken inside columns, left a last one of 44 lanes and
     // lines stored in two parts: P3^3 elasticity, 100,003 tets, FP64 692 -> 563 us
-    // (5.1 TB/s), FP32 458 -> 378 us
+    // (5.1 TB/s), FP32 458 -> 378 us.  Fewer columns where a group of all of them
+    // would leave a quarter of the lanes idle (P2^3 against P3^3: 150 of 256)
     const int nfB = a.nfB0 * NCB, rows = nfB / VEC;
     const T* R = reinterpret_cast<const T*>(
         sizeof(T) == 8 ? static_cast<const void*>(SYM ? a.Rds : a.Rd) : static_cast<const void*>(SYM ? a.Rfs : a.Rf));
@@ -120,6 +121,7 @@ __global__ __launch_bounds__(kBlock) void element_const_kernel(ElemArgs a) {
     for (int c0 = 0, C; c0 < a.nfA0; c0 += J * C) {
         C = (a.nfA0 - c0 + J - 1) / J;
         if (C > kBlock / rows) C = kBlock / rows;
+        while (C > 1 && rows * C * (kBlock / (rows * C)) < 3 * kBlock / 4) --C;
         const int L = rows * C, NG = kBlock / L, g = threadIdx.x / L, item = threadIdx.x - g * L;
         if (g >= NG) continue;
         const int c = c0 + item / rows, ib = VEC * (item % rows), cb = ib / a.nfB0, ib0 = ib - cb * a.nfB0;

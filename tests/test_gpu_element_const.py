@@ -67,7 +67,9 @@ def test_const_kernel_shapes_match_oracle(pair, tt, n):
 @pytest.mark.parametrize("pair,tt,n", [
     ((2, 4, 3, 2, 4, 3), af.TENSOR_GENERAL, 1), ((1, 4, 3, 1, 4, 3), af.TENSOR_SCALAR, 37),
     ((2, 4, 3, 2, 4, 3), af.TENSOR_SYMMETRIC, 512 * 32 + 1), ((1, 4, 1, 2, 4, 3), af.TENSOR_GENERAL, 51),
-    ((2, 4, 3, 1, 4, 1), af.TENSOR_GENERAL, 49), ((2, 3, 1, 2, 4, 3), af.TENSOR_GENERAL, 18)])
+    ((2, 4, 3, 1, 4, 1), af.TENSOR_GENERAL, 49), ((2, 3, 1, 2, 4, 3), af.TENSOR_GENERAL, 18),
+    ((2, 3, 3, 2, 4, 3), af.TENSOR_GENERAL, 41), ((2, 4, 3, 2, 3, 3), af.TENSOR_GENERAL, 41),
+    ((1, 3, 3, 1, 4, 3), af.TENSOR_SCALAR, 1)])
 def test_matrices_of_several_passes_match_oracle(pair, tt, n):
     """More items than lanes: whole columns per pass, the last pass's cells dealt
     out to groups of lanes."""
@@ -75,7 +77,7 @@ def test_matrices_of_several_passes_match_oracle(pair, tt, n):
 
 
 @pytest.mark.parametrize("pair,tt", [((1, 21, 1, 1, 21, 1), af.TENSOR_GENERAL), ((2, 25, 1, 2, 25, 1), af.TENSOR_SYMMETRIC),
-                                     ((4, 25, 1, 4, 25, 1), af.TENSOR_GENERAL)])
+                                     ((4, 25, 1, 4, 25, 1), af.TENSOR_GENERAL), ((1, 4, 3, 1, 21, 1), af.TENSOR_GENERAL)])
 @pytest.mark.parametrize("n", [384 * 32 - 1, 384 * 32, 384 * 128 + 5, 384 * 256 - 1, 384 * 256 + 1])
 def test_face_and_edge_spaces_either_side_of_a_change_of_cells_per_workgroup(pair, tt, n):
     test_const_kernel_shapes_match_oracle(pair, tt, n)
